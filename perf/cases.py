@@ -1,0 +1,482 @@
+"""The work that users of this framework have it do, as timed cases.
+
+Six kinds, each through the entry points a program calls:
+
+  fdm      GpuDogfight: an episode segment of the batched flight model (load a seed, then one
+           `step` per decision), fp64 or fp32, with or without the 17-value output;
+  env      GpuDogfightVecEnv.step: one decision of the full environment (physics, observation,
+           reward, termination, autoreset);
+  policy   PolicyStep: the per-step inference of a collector -- the learner (RunningNorm.update,
+           then both heads with every rollout output) or a league's frozen opponents (grouped
+           networks, row map, device-side group offsets);
+  gae      advantages and returns over a rollout buffer;
+  ppo      one minibatch of the PPO update: PPOUpdater.minibatch_grad and optimizer_step;
+  rollout  SelfPlayRollout / LeagueRollout.collect: a whole rollout, recorded as a HIP graph and
+           replayed.
+
+Sizes span what the framework is run with: 64 engagements (the head-on evaluation set) to 65,536
+(league scale), 184- and 214-wide observations, odd counts in between.
+"""
+import importlib
+import math
+import os
+import sys
+
+import numpy as np
+import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+if ROOT not in sys.path:
+    sys.path.insert(0, ROOT)
+PKG = "2026_ai_pilot_challenge-1st_solution_amd"
+DEVICE = "cuda"
+SUBSTEPS = 6
+DECISIONS = 20                      # of an fdm episode segment
+
+
+def _mod(name=""):
+    return importlib.import_module(PKG + name)
+
+
+# ---------------------------------------------------------------- the cases
+def listed():
+    return [
+        # the head-on evaluation set watched by a program that reads the 17-value output after
+        # every decision: the smallest batch, bound by latency and launches
+        {"name": "fdm_headon_64", "kind": "fdm", "nenv": 64, "precision": "fp64", "rate": 120,
+         "obs": True},
+        # the flight model at the batch size of the framework's headline figure
+        {"name": "fdm_tailchase_16k", "kind": "fdm", "nenv": 16384, "precision": "fp64",
+         "rate": 120, "obs": False},
+        # the single-precision option at the same size
+        {"name": "fdm_tailchase_16k_fp32", "kind": "fdm", "nenv": 16384, "precision": "fp32",
+         "rate": 120, "obs": False},
+        # a development run: an odd number of engagements, the wide observation
+        {"name": "env_777_214", "kind": "env", "nenv": 777, "obs_dim": 214},
+        # the training environment at its usual size
+        {"name": "env_16k_184", "kind": "env", "nenv": 16384, "obs_dim": 184},
+        # league scale
+        {"name": "env_64k_214", "kind": "env", "nenv": 65536, "obs_dim": 214},
+        # the self-play learner's inference: both aircraft of 16,384 engagements
+        {"name": "policy_learner_32k_184", "kind": "policy", "rows": 32768, "obs_dim": 184,
+         "nets": 1},
+        # the league's eight opponents, one plane of 65,536 engagements
+        {"name": "policy_league_64k_214", "kind": "policy", "rows": 65536, "obs_dim": 214,
+         "nets": 8},
+        # advantages of a self-play rollout
+        {"name": "gae_64x16k", "kind": "gae", "T": 64, "nenv": 16384, "agents": 2},
+        # a minibatch of a small run (ragged against the 64-row tiles), with the entropy bonus
+        {"name": "ppo_5000_214", "kind": "ppo", "rows": 5000, "obs_dim": 214, "ent_coef": 0.01},
+        # a minibatch of the self-play update: 64 x 32,768 transitions in 8 minibatches
+        {"name": "ppo_256k_184", "kind": "ppo", "rows": 262144, "obs_dim": 184, "ent_coef": 0.0},
+        # the whole self-play rollout
+        {"name": "rollout_16k_T64", "kind": "rollout", "nenv": 16384, "T": 64, "opponents": 0},
+    ]
+
+
+def _spread(rng, lo, hi):
+    """A size spread over the logarithm of [lo, hi]; half of them a multiple of 64."""
+    n = int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+    if rng.random() < 0.5 and n >= 128:
+        n = n // 64 * 64
+    return max(lo, min(hi, n))
+
+
+def draw(rng):
+    kind = rng.choice(["fdm", "env", "policy", "gae", "ppo", "rollout"])
+    dim = rng.choice([184, 214])
+    if kind == "fdm":
+        return {"kind": kind, "nenv": _spread(rng, 16, 65536),
+                "precision": rng.choice(["fp64", "fp64", "fp32"]), "rate": rng.choice([120, 60]),
+                "obs": rng.random() < 0.5}
+    if kind == "env":
+        return {"kind": kind, "nenv": _spread(rng, 16, 65536), "obs_dim": dim}
+    if kind == "policy":
+        return {"kind": kind, "rows": _spread(rng, 32, 65536), "obs_dim": dim,
+                "nets": rng.choice([1, 1, 4, 8])}
+    if kind == "gae":
+        return {"kind": kind, "T": rng.randint(8, 128), "nenv": _spread(rng, 64, 65536),
+                "agents": rng.choice([1, 2])}
+    if kind == "ppo":
+        return {"kind": kind, "rows": _spread(rng, 256, 262144), "obs_dim": dim,
+                "ent_coef": rng.choice([0.0, 0.01])}
+    nenv = _spread(rng, 64, 16384)
+    return {"kind": kind, "nenv": nenv, "T": rng.randint(8, 64), "opponents": rng.choice([0, 0, 8])}
+
+
+# ---------------------------------------------------------------- inputs
+def _gen(seed):
+    return torch.Generator(device=DEVICE).manual_seed(int(seed))
+
+
+def _bin_actions(shape, gen, dtype):
+    """Uniform draws of the 21-bin controls (throttle in [0, 1]) on the device."""
+    idx = torch.randint(0, 21, (*shape, 4), generator=gen, device=DEVICE)
+    a = torch.linspace(-1.0, 1.0, 21, dtype=torch.float64, device=DEVICE)[idx]
+    a[..., 3] = 0.5 * a[..., 3] + 0.5
+    return a.to(dtype).contiguous()
+
+
+def _observations(rows, dim, gen):
+    """Raw observation rows: every column with a mean and a spread of its own, as the
+    observation's blocks (scaled angles, distances, tanh and Gaussian features) have."""
+    mean = torch.randn(dim, generator=gen, device=DEVICE) * 0.5
+    spread = torch.rand(dim, generator=gen, device=DEVICE) * 0.9 + 0.1
+    x = torch.randn(rows, dim, generator=gen, device=DEVICE)
+    return (x * spread + mean).contiguous()
+
+
+def _net(dim, seed, init="normal"):
+    net = _mod(".policy").MLPActorCritic(dim, init=init, init_std=0.02,
+                                         generator=torch.Generator().manual_seed(int(seed)))
+    return net.to(DEVICE)
+
+
+def _group_sizes(rows, nets):
+    """Rows per opponent: Zipf(1.1) weights, as the league assigns them."""
+    w = np.array([float(k + 1) ** -1.1 for k in range(nets)])
+    cut = np.floor(np.cumsum(w / w.sum()) * rows).astype(np.int64)
+    cut[-1] = rows
+    return np.diff(np.concatenate([[0], cut]))
+
+
+def prepare(case, seed):
+    return {"fdm": _prepare_fdm, "env": _prepare_env, "policy": _prepare_policy,
+            "gae": _prepare_gae, "ppo": _prepare_ppo,
+            "rollout": _prepare_rollout}[case["kind"]](case, int(seed))
+
+
+def _prepare_fdm(case, seed):
+    ic = _mod(".ic")
+    sim = _mod().GpuDogfight(case["nenv"], substeps=SUBSTEPS, precision=case["precision"],
+                             fcs_rate=case["rate"], device=DEVICE)
+    rows = (ic.sample_headon if case["nenv"] <= 64 else ic.sample_tailchase)(case["nenv"], seed)
+    sim.seed_rows(torch.as_tensor(rows, device=DEVICE))
+    return {"case": case, "sim": sim, "seed": sim.states.double().clone(),
+            "actions": _bin_actions((DECISIONS, sim.nac), _gen(seed), sim.dtype)}
+
+
+def _prepare_env(case, seed):
+    env = _mod(".rl_env").GpuDogfightVecEnv(case["nenv"], seed=seed, obs_dim=case["obs_dim"],
+                                            device=DEVICE)
+    env.reset()
+    return {"case": case, "env": env, "k": 0,
+            "actions": _bin_actions((8, env.nac), _gen(seed), torch.float64)}
+
+
+def _prepare_policy(case, seed):
+    pol = _mod(".policy")
+    dim, rows, nets = case["obs_dim"], case["rows"], case["nets"]
+    g = _gen(seed)
+    phys = rows if nets == 1 else 2 * rows          # a league's opponents fly plane 1
+    st = {"case": case, "step": pol.PolicyStep(dim, DEVICE, seed=seed),
+          "obs": _observations(phys, dim, g),
+          "env_actions": torch.zeros(phys, 4, dtype=torch.float64, device=DEVICE),
+          "logits": torch.empty(rows, 84, device=DEVICE)}
+    if nets == 1:
+        st["net"], st["norm"] = _net(dim, seed), pol.RunningNorm(dim, DEVICE)
+        st["net"].pack()
+        st["nobs"] = torch.empty(rows, dim, device=DEVICE)
+        st["act"] = torch.empty(rows, 4, dtype=torch.int64, device=DEVICE)
+        st["logp"], st["value"] = (torch.empty(rows, device=DEVICE) for _ in range(2))
+        return st
+    sizes = _group_sizes(rows, nets)
+    perm = torch.randperm(rows, generator=g, device=DEVICE)
+    order = torch.cat([p.sort().values for p in perm.split(sizes.tolist())])
+    st["rows"] = (2 * order + 1).to(torch.int32)
+    st["offsets"] = torch.as_tensor(np.concatenate([[0], np.cumsum(sizes)]), dtype=torch.int32,
+                                    device=DEVICE)
+    st["groups"] = []
+    for k in range(nets):
+        norm = pol.RunningNorm(dim, DEVICE)
+        norm.mean.copy_(torch.randn(dim, generator=g, device=DEVICE) * 0.5)
+        norm.var.copy_((torch.rand(dim, generator=g, device=DEVICE) * 0.9 + 0.1) ** 2)
+        net = _net(dim, 1000 * (seed % 1000000) + k)
+        net.pack()
+        st["groups"].append((net, None, None, norm))
+    return st
+
+
+def _prepare_gae(case, seed):
+    T, ne, na = case["T"], case["nenv"], case["agents"]
+    g = _gen(seed)
+    shape = (T, ne, na) if na > 1 else (T, ne)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEVICE)
+    return {"case": case, "rew": r(*shape) * 0.1, "val": r(*shape),
+            "done": (torch.rand(T, ne, generator=g, device=DEVICE) < 0.005).float(),
+            "last_val": r(*shape[1:]),
+            "next_done": (torch.rand(ne, generator=g, device=DEVICE) < 0.005).float()}
+
+
+def _prepare_ppo(case, seed):
+    up = _mod(".ppo_update")
+    dim, rows = case["obs_dim"], case["rows"]
+    count = 2 * rows                                # the minibatch is drawn from a rollout
+    g = _gen(seed)
+    net = _net(dim, seed, init="orthogonal")
+    obs = torch.randn(count, dim, generator=g, device=DEVICE).clamp(-10, 10)
+    # the collection policy's draws and log-probabilities, moved a little since
+    with torch.no_grad():
+        lsm = torch.log_softmax(net.forward_reference(obs)[0], dim=-1)
+        u = torch.rand(count, 4, 1, generator=g, device=DEVICE)
+        act = (lsm.exp().cumsum(-1) < u).sum(-1).clamp(max=20)
+        logp = lsm.gather(-1, act.unsqueeze(-1)).squeeze(-1).sum(-1)
+        logp += 0.1 * torch.randn(count, generator=g, device=DEVICE)
+    r = lambda: torch.randn(count, generator=g, device=DEVICE)
+    return {"case": case, "obs": obs, "act": act, "logp": logp, "adv": r(), "ret": r(),
+            "idx": torch.randperm(count, generator=g, device=DEVICE)[:rows].contiguous(),
+            "up": up.PPOUpdater(net, up.UpdateConfig(ent_coef=case["ent_coef"]), seed=seed)}
+
+
+def _prepare_rollout(case, seed):
+    ppo, env_mod = _mod(".ppo"), _mod(".rl_env")
+    if case["opponents"]:
+        env = env_mod.GpuDogfightVecEnv(case["nenv"], seed=seed, obs_dim=214, device=DEVICE,
+                                        fuel_exhaustion=True, fuel_lbs_range=(100.0, 3000.0))
+        opps = [_net(214, 100 + k) for k in range(case["opponents"])]
+        ro = ppo.LeagueRollout(env, _net(214, seed), opps, T=case["T"], seed=seed, graph=True)
+    else:
+        env = env_mod.GpuDogfightVecEnv(case["nenv"], seed=seed, device=DEVICE)
+        ro = ppo.SelfPlayRollout(env, _net(184, seed), T=case["T"], seed=seed, stats=False,
+                                 graph=True)
+    ro.reset()
+    return {"case": case, "ro": ro}
+
+
+# ---------------------------------------------------------------- one pass
+def _state_parts(states):
+    """The (nac, 101) state by quantity, so that each is compared at its own scale."""
+    cuts = {"position": (0, 3), "velocity": (3, 6), "attitude": (6, 10), "rates": (10, 13),
+            "fuel": (14, 15), "accelerations": (15, 25), "rate_history": (25, 46),
+            "velocity_history": (46, 55), "acceleration_history": (55, 64),
+            "previous": (64, 82), "engine": (82, 86), "actuators": (86, 92), "pid": (92, 101)}
+    return {k: states[:, a:b] for k, (a, b) in cuts.items()}
+
+
+def run(state):
+    case = state["case"]
+    kind = case["kind"]
+    if kind == "fdm":
+        sim, acts = state["sim"], state["actions"]
+        sim.load_seed(state["seed"])
+        for k in range(DECISIONS):
+            out = sim.step(acts[k], want_obs=case["obs"])
+        got = _state_parts(sim.states)
+        if case["obs"]:
+            o = out.reshape(sim.nac, -1)
+            got.update(out_euler=o[:, 6:9], out_uvw=o[:, 9:12], out_alpha_beta=o[:, 12:14],
+                       out_mach=o[:, 14:15], out_vt=o[:, 15:16], out_alt=o[:, 16:17])
+        return got
+    if kind == "env":
+        env = state["env"]
+        acts = state["actions"][state["k"] % 8]
+        state["k"] += 1
+        obs, reward, done, info = env.step(acts)
+        return {"obs": obs, "reward": reward, "done": done, "hp": env.obr.hp,
+                **{k: info[k] for k in ("terminated", "truncated", "terminal_obs", "terminal_hp",
+                                        "terminal_alt_m", "terminal_state_finite")},
+                **_state_parts(env.sim.states)}
+    if kind == "policy":
+        st = state
+        if case["nets"] == 1:
+            st["norm"].update(st["obs"])
+            st["step"](st["obs"], [(st["net"], 0, case["rows"])], norm=st["norm"],
+                       nobs_out=st["nobs"], act_idx=st["act"], logp=st["logp"],
+                       value=st["value"], env_actions=st["env_actions"], logits_out=st["logits"])
+            return {"mean": st["norm"].mean, "var": st["norm"].var, "nobs": st["nobs"],
+                    "act": st["act"], "logp": st["logp"], "value": st["value"],
+                    "env_actions": st["env_actions"], "logits": st["logits"]}
+        st["step"](st["obs"], st["groups"], rows=st["rows"], group_offsets=st["offsets"],
+                   max_group_rows=case["rows"], nphys=2 * case["rows"], salt=1,
+                   env_actions=st["env_actions"], logits_out=st["logits"])
+        return {"env_actions": st["env_actions"], "logits": st["logits"]}
+    if kind == "gae":
+        adv, ret = _mod(".ppo").gae(state["rew"], state["val"], state["done"], state["last_val"],
+                                    state["next_done"], 0.99, 0.95)
+        return {"adv": adv, "ret": ret}
+    if kind == "ppo":
+        up = state["up"]
+        up.minibatch_grad(state["obs"], state["act"], state["logp"], state["adv"], state["ret"],
+                          state["idx"])
+        up.optimizer_step()
+        return {"grad": up.grad, "weights": up.flat, "exp_avg": up.exp_avg,
+                "exp_avg_sq": up.exp_avg_sq, "grad_norms": up.grad_norms, "stats": up.stats[0]}
+    ro = state["ro"]
+    adv, ret, _ = ro.collect()
+    return {"obs": ro.b_obs, "act": ro.b_act, "logp": ro.b_logp, "value": ro.b_val,
+            "reward": ro.b_rew, "done": ro.b_done, "adv": adv, "ret": ret,
+            "last_value": ro.last_val, "norm_mean": ro.norm.mean, "norm_var": ro.norm.var}
+
+
+# ---------------------------------------------------------------- what a pass cannot do without
+FLOP_SUBSTEP = 1550                  # arithmetic of one aircraft-substep (counted, fp64 model)
+# one aircraft's decision: 66 state values read and 101 written, 4 controls
+FDM_VALUES = 66 + 101 + 4
+# the rest of an environment step: reconstructor, reward, flags and the two observation rows
+POST_VALUES = (4 + 27) + (34 + 3)
+
+
+def _mlp_flops(dim, critic=True):
+    return 2 * ((2 if critic else 1) * (256 * dim + 256 * 256) + 84 * 256 + (256 if critic else 0))
+
+
+def _env_work(nac, dim):
+    post = POST_VALUES * 8 + 2 * dim * 4 + (72 if dim == 214 else 0)
+    return {"bytes": nac * (FDM_VALUES * 8 + post), "flops": nac * SUBSTEPS * FLOP_SUBSTEP}
+
+
+def work(case):
+    kind = case["kind"]
+    if kind == "fdm":
+        nac, w = 2 * case["nenv"], 8 if case["precision"] == "fp64" else 4
+        values = FDM_VALUES + (17 if case["obs"] else 0)
+        return {"bytes": DECISIONS * nac * w * values,
+                "flops": DECISIONS * nac * SUBSTEPS * FLOP_SUBSTEP}
+    if kind == "env":
+        return _env_work(2 * case["nenv"], case["obs_dim"])
+    if kind == "policy":
+        dim, rows, one = case["obs_dim"], case["rows"], case["nets"] == 1
+        per = dim * 4 + 32 + 84 * 4 + (dim * 4 + 32 + 8 if one else 4)
+        weights = (2 if one else 1) * (256 * dim + 256 * 256) * 2 + 84 * 256 * 2
+        return {"bytes": rows * per + case["nets"] * weights, "flops": rows * _mlp_flops(dim, one)}
+    if kind == "gae":
+        n = case["T"] * case["nenv"]
+        return {"bytes": 4 * n * (4 * case["agents"] + 1), "flops": 7 * n * case["agents"]}
+    if kind == "ppo":
+        dim, rows = case["obs_dim"], case["rows"]
+        params = 2 * (256 * dim + 256 * 256 + 512) + 85 * 256 + 85
+        flops = rows * (2 * _mlp_flops(dim) + 2 * (84 * 256 + 2 * 256 * 256 + 256))
+        return {"bytes": rows * (dim * 4 + 32 + 12 + 8) + params * (7 * 4 + 4), "flops": flops}
+    T, ne, league = case["T"], case["nenv"], bool(case["opponents"])
+    dim = 214 if league else 184
+    rows = ne if league else 2 * ne
+    step = _env_work(2 * ne, dim)
+    # the step writes no terminal rows; the learner reads its rows and writes the normalised ones
+    by = step["bytes"] - 2 * ne * dim * 4 + rows * (2 * dim * 4 + 32 + 8 + 32)
+    fl = step["flops"] + rows * _mlp_flops(dim)
+    if league:
+        by += ne * (dim * 4 + 32)
+        fl += ne * _mlp_flops(dim, critic=False)
+    return {"bytes": T * (by + rows * 16), "flops": T * fl}
+
+
+# ---------------------------------------------------------------- how far results may lie apart
+def tolerance(case):
+    kind = case["kind"]
+    if kind == "fdm":
+        return FDM_TOLERANCE[case["precision"]]
+    return TOLERANCE[kind]
+
+
+# fp64 flight model: 20 decisions against the CPU restatement (1.3e-14, 2.6e-13).  fp32: the float
+# build against the fp64 restatement (2.4e-3, 0.1 at most).  Policy, update and rollout: the same
+# networks with their hidden units in another order, and the minibatch's rows in another order.
+# A draw that falls on the other side of a bin's edge moves that control by one bin, and in a
+# rollout the trajectory that follows.
+FDM_TOLERANCE = {"fp64": {"rel": 1e-12, "max": 1e-11}, "fp32": {"rel": 1e-2, "max": 0.4}}
+TOLERANCE = {
+    "env": {"rel": 1e-6, "max": 1e-4, "differ": 1e-4},
+    "policy": {"rel": 1e-4, "max": 0.3, "differ": 1e-4},
+    "gae": {"rel": 2e-6, "max": 1e-5},
+    "ppo": {"rel": 4e-4, "max": 1e-2},
+    "rollout": {"rel": 1e-3, "max": 0.9, "differ": 1e-3},
+}
+
+
+# ---------------------------------------------------------------- the same results in 64 bits
+def exact(case, seed):
+    """Plain torch in float64.  None for the flight model and what contains it: the model is
+    fp64 arithmetic already, and has no shorter statement than its own source."""
+    if case["kind"] == "policy":
+        return _exact_policy(prepare(case, seed))
+    if case["kind"] == "gae":
+        return _exact_gae(prepare(case, seed))
+    if case["kind"] == "ppo":
+        return _exact_ppo(prepare(case, seed))
+    return None
+
+
+def _linears(seq):
+    return [(m.weight.detach().double(), m.bias.detach().double()) for m in seq
+            if hasattr(m, "weight")]
+
+
+def _forward(layers, x):
+    for w, b in layers[:-1]:
+        x = torch.tanh(x @ w.t() + b)
+    return x @ layers[-1][0].t() + layers[-1][1]
+
+
+def _normalised(x, mean, var):
+    return ((x - mean) / torch.sqrt(var + 1e-8)).clamp(-10.0, 10.0)
+
+
+def _exact_policy(st):
+    case = st["case"]
+    if case["nets"] == 1:
+        x = st["obs"].double()
+        n0, n = 1e-4, float(case["rows"])
+        mu, v = x.mean(0), x.var(0, correction=0)
+        tot = n0 + n
+        mean = mu * (n / tot)
+        var = (n0 + v * n + mu * mu * (n0 * n / tot)) / tot
+        nobs = _normalised(x, mean, var)
+        net = st["net"]
+        return {"mean": mean, "var": var, "nobs": nobs, "act": None, "logp": None,
+                "value": _forward(_linears(net.critic), nobs).squeeze(-1), "env_actions": None,
+                "logits": _forward(_linears(net.actor_logits), nobs)}
+    cuts = st["offsets"].tolist()
+    out = []
+    for k, (net, _, _, norm) in enumerate(st["groups"]):
+        x = st["obs"][st["rows"][cuts[k]:cuts[k + 1]].long()].double()
+        out.append(_forward(_linears(net.actor_logits),
+                            _normalised(x, norm.mean.double(), norm.var.double())))
+    return {"env_actions": None, "logits": torch.cat(out)}
+
+
+def _exact_gae(st):
+    rew, val = st["rew"].double(), st["val"].double()
+    T = rew.shape[0]
+    expand = lambda d: d.double() if rew.dim() == 2 else d.double().unsqueeze(-1)
+    adv = torch.empty_like(rew)
+    last = torch.zeros_like(rew[0])
+    for t in reversed(range(T)):
+        nd = expand(st["next_done"] if t == T - 1 else st["done"][t + 1])
+        nv = st["last_val"].double() if t == T - 1 else val[t + 1]
+        last = rew[t] + 0.99 * nv * (1 - nd) - val[t] + 0.99 * 0.95 * (1 - nd) * last
+        adv[t] = last
+    return {"adv": adv, "ret": adv + val}
+
+
+def _exact_ppo(st):
+    cfg, net = st["up"].cfg, st["up"].net
+    idx = st["idx"]
+    obs, ret = st["obs"][idx].double(), st["ret"][idx].double()
+    act, old, adv = st["act"][idx], st["logp"][idx].double(), st["adv"][idx].double()
+    params = [p for seq in (net.actor_logits, net.critic) for m in seq if hasattr(m, "weight")
+              for p in (m.weight, m.bias)]
+    params = [p.detach().double().clone().requires_grad_(True) for p in params]
+    layers = [(params[2 * i], params[2 * i + 1]) for i in range(6)]
+    lsm = torch.log_softmax(_forward(layers[:3], obs).view(-1, 4, 21), dim=-1)
+    new = lsm.gather(-1, act.unsqueeze(-1)).squeeze(-1).sum(-1)
+    ent = -(lsm.exp() * lsm).sum(-1).sum(-1).mean()
+    log_ratio = new - old
+    ratio = log_ratio.exp()
+    a = (adv - adv.mean()) / (adv.std() + 1e-8)
+    pl = torch.max(-a * ratio, -a * ratio.clamp(1 - cfg.clip_coef, 1 + cfg.clip_coef)).mean()
+    vl = 0.5 * ((_forward(layers[3:], obs).squeeze(-1) - ret) ** 2).mean()
+    (pl - cfg.ent_coef * ent + cfg.vf_coef * vl).backward()
+    grad = [p.grad.reshape(-1) for p in params]
+    actor, critic = torch.cat(grad[:6]), torch.cat(grad[6:])
+    norms = torch.stack([actor.norm(), critic.norm()])
+    scale = (cfg.max_grad_norm / (norms + 1e-6)).clamp(max=1.0)
+    clipped = torch.cat([actor * scale[0], critic * scale[1]])
+    m, v = 0.1 * clipped, 0.001 * clipped * clipped
+    flat = torch.cat([p.detach().reshape(-1) for p in params])
+    weights = flat - cfg.lr / (1 - 0.9) * m / (v.sqrt() / math.sqrt(1 - 0.999) + 1e-5)
+    kl = ((ratio - 1.0) - log_ratio).mean()
+    cf = ((ratio - 1.0).abs() > cfg.clip_coef).double().mean()
+    stats = torch.stack([pl.detach(), vl.detach(), ent.detach(), kl.detach(), cf, adv.mean(),
+                         adv.std(), torch.zeros_like(cf)])
+    return {"grad": torch.cat([actor, critic]), "weights": weights, "exp_avg": m, "exp_avg_sq": v,
+            "grad_norms": norms, "stats": stats}
