@@ -478,5 +478,5 @@ def _exact_ppo(st):
     cf = ((ratio - 1.0).abs() > cfg.clip_coef).double().mean()
     stats = torch.stack([pl.detach(), vl.detach(), ent.detach(), kl.detach(), cf, adv.mean(),
                          adv.std(), torch.zeros_like(cf)])
-    return {"grad": torch.cat([actor, critic]), "weights": weights, "exp_avg": m, "exp_avg_sq": v,
+    return {"grad": clipped, "weights": weights, "exp_avg": m, "exp_avg_sq": v,
             "grad_norms": norms, "stats": stats}
