@@ -290,7 +290,10 @@ F16_HD Mass mass_props(double fuel) {
 }
 
 // Pitot total pressure and its inverse (jsb_auxiliary.py:20-42) -> calibrated airspeed, ft/s.
-F16_HD double vcal_from_mach(double mach, double p) {
+// `refine` (wave-uniform) false leaves a supersonic result at the subsonic inverse's value, which
+// is above Mach 1 as the refined one is (A >= 1.893 there, and each pass maps M >= 1 to M >= 1):
+// enough for a caller that only compares the airspeed with speeds far below Mach 1.
+F16_HD double vcal_from_mach(double mach, double p, bool refine = true) {
   double pt;
   if (mach < 0.0) {
     pt = p;
@@ -304,7 +307,7 @@ F16_HD double vcal_from_mach(double mach, double p) {
   const double qc = pt - p;
   const double A = qc * (1.0 / 2116.228) + 1.0;  // StdDaySLpressure (jsb_const.py:24)
   double M = fm_sqrt(5.0 * (fm_exp(fm_log(A) * (1.0 / 3.5)) - 1.0));
-  if (M > 1.0) {
+  if (refine && M > 1.0) {
     for (int i = 0; i < 10; ++i) {
       const double t = 1.0 - fm_rcp(7.0 * M * M);
       M = 0.8812848543473311 * fm_sqrt(A * (t * t * fm_sqrt(t)));
@@ -338,12 +341,13 @@ F16_HD void body_dcm(const double q[4], double B[3][3]) {
   B[2][0] = 2.0 * (q1q3 + q0q2); B[2][1] = 2.0 * (q2q3 - q0q1); B[2][2] = q0q0 - q1q1 - q2q2 + q3q3;
 }
 
-// `want_euler` (wave-uniform) also produces the Euler angles (mat_to_euler,
-// jsb_frames.py:140-163) for the output row; the FCS only needs cos(theta)cos(phi), which is
-// formed from the DCM without the inverse trigonometry.
-F16_HD void kinematics(const double p[3], const double v[3], const double q[4],
-                       const double wi[3], double ce, double se, bool want_euler, Kin& k,
-                       double euler[3]) {
+// The half of the frames that position and attitude alone decide (a cooperating wavefront forms
+// it a phase before the velocity exists): everything in `k` but uvw, wpqr, vn and ve, and the
+// body axes in the local frame, L[i][j] = body_i . local_j.  `want_euler` (wave-uniform) also
+// produces the Euler angles (mat_to_euler, jsb_frames.py:140-163) for the output row; the FCS
+// only needs cos(theta)cos(phi), which is formed from the DCM without the inverse trigonometry.
+F16_HD void kin_pose(const double p[3], const double q[4], double ce, double se, bool want_euler,
+                     Kin& k, double L[3][3], double euler[3]) {
   k.ce = ce;
   k.se = se;
   k.ex = ce * p[0] + se * p[1];
@@ -366,26 +370,18 @@ F16_HD void kinematics(const double p[3], const double v[3], const double q[4],
   const double D[3] = {ce * d0 - se * d1, se * d0 + ce * d1, -sLat};
   body_dcm(q, k.B);
   // Tl2b[i][j] = body_i . local_j
-  double L[3][3];
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     L[i][0] = k.B[i][0] * N[0] + k.B[i][1] * N[1] + k.B[i][2] * N[2];
     L[i][1] = k.B[i][0] * E[0] + k.B[i][1] * E[1];
     L[i][2] = k.B[i][0] * D[0] + k.B[i][1] * D[1] + k.B[i][2] * D[2];
   }
-  // body velocity relative to the rotating Earth: Ti2b (v - omega x p)
-  const double dv[3] = {v[0] + kRot * p[1], v[1] - kRot * p[0], v[2]};
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    k.uvw[i] = k.B[i][0] * dv[0] + k.B[i][1] * dv[1] + k.B[i][2] * dv[2];
-    k.wpqr[i] = wi[i] - k.B[i][2] * kRot;   // vPQR = vPQRi - Ti2b * omega
-  }
-  k.vn = L[0][0] * k.uvw[0] + L[1][0] * k.uvw[1] + L[2][0] * k.uvw[2];
-  k.ve = L[0][1] * k.uvw[0] + L[1][1] * k.uvw[1] + L[2][1] * k.uvw[2];
   const double d6 = L[0][2];
   const bool gimbal = d6 <= -1.0 || d6 >= 1.0;
   if (gimbal) {
-    k.ctcp = 6.123233995736766e-17 * cos(atan2(-L[2][1], L[1][1]));   // cos(+-pi/2) in double
+    // cos(+-pi/2) in double times cos(atan2(-L21, L11)), the latter as its vector ratio
+    const double h = fm_sqrt(L[1][1] * L[1][1] + L[2][1] * L[2][1]);
+    k.ctcp = 6.123233995736766e-17 * (h != 0.0 ? fm_div(L[1][1], h) : 1.0);
   } else {
     const double h = fm_sqrt(L[1][2] * L[1][2] + L[2][2] * L[2][2]);
     k.ctcp = fm_sqrt(1.0 - d6 * d6) * (h != 0.0 ? fm_div(L[2][2], h) : 1.0);
@@ -402,6 +398,28 @@ F16_HD void kinematics(const double p[3], const double v[3], const double q[4],
       euler[2] = ps < 0.0 ? ps + 2.0 * M_PI : ps;
     }
   }
+}
+
+// Body velocity relative to the rotating Earth, Ti2b (v - omega x p), and the body rates
+// relative to it, vPQR = vPQRi - Ti2b * omega.
+F16_HD void body_motion(const double B[3][3], const double p[3], const double v[3],
+                        const double wi[3], double uvw[3], double wpqr[3]) {
+  const double dv[3] = {v[0] + kRot * p[1], v[1] - kRot * p[0], v[2]};
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    uvw[i] = B[i][0] * dv[0] + B[i][1] * dv[1] + B[i][2] * dv[2];
+    wpqr[i] = wi[i] - B[i][2] * kRot;
+  }
+}
+
+F16_HD void kinematics(const double p[3], const double v[3], const double q[4],
+                       const double wi[3], double ce, double se, bool want_euler, Kin& k,
+                       double euler[3]) {
+  double L[3][3];
+  kin_pose(p, q, ce, se, want_euler, k, L, euler);
+  body_motion(k.B, p, v, wi, k.uvw, k.wpqr);
+  k.vn = L[0][0] * k.uvw[0] + L[1][0] * k.uvw[1] + L[2][0] * k.uvw[2];
+  k.ve = L[0][1] * k.uvw[0] + L[1][1] * k.uvw[1] + L[2][1] * k.uvw[2];
 }
 
 // ------------------------------------------------------------------ force path components
@@ -534,15 +552,15 @@ F16_HD void load_factors(const Aircraft& a, const double cg[3], double& npy, dou
   npz = (a.pba[2] + c1z + c3z) * (1.0 / F16M_SLGRAVITY);
 }
 
-F16_HD double vc_knots(double mach, double P) {
-  return (fabs(mach) > 0.0) ? vcal_from_mach(mach, P) * F16M_FPSTOKTS : 0.0;
+F16_HD double vc_knots(double mach, double P, bool refine = true) {
+  return (fabs(mach) > 0.0) ? vcal_from_mach(mach, P, refine) * F16M_FPSTOKTS : 0.0;
 }
 
 // ---- engine (jsb_propulsion.py:89-128); throttle position = 2 * throttle command ----
-// Updates the spool and fuel-flow state in `a`; returns the thrust, and the fuel burnt this
+// engine_spool moves the spool speeds in `a` (no Mach number needed) and returns the augmentation
+// position; engine_thrust updates the fuel flow and returns the thrust, and the fuel burnt this
 // step in `burn`.
-F16_HD double engine(Aircraft& a, double c_thr, const Atmos& at, double mach,
-                     const double* __restrict__ T, double& burn) {
+F16_HD double engine_spool(Aircraft& a, double c_thr, const Atmos& at) {
   double thr = 2.0 * c_thr, aug = 0.0;
   if (thr > 1.0) { aug = thr - 1.0; thr -= aug; }
   // spool-time constants as the reference forms them: k * 90 / (bypass + 3)
@@ -557,6 +575,11 @@ F16_HD double engine(Aircraft& a, double c_thr, const Atmos& at, double mach,
   a.n2 = seek(a.n2, F16M_ENG_IDLEN2 + thr * (F16M_ENG_MAXN2 - F16M_ENG_IDLEN2), up, n2dn);
   a.n1 = seek(a.n1, F16M_ENG_IDLEN1 + thr * (F16M_ENG_MAXN1 - F16M_ENG_IDLEN1), up, n1dn);
   a.n2n = (a.n2 - F16M_ENG_IDLEN2) * (1.0 / (F16M_ENG_MAXN2 - F16M_ENG_IDLEN2));
+  return aug;
+}
+
+F16_HD double engine_thrust(Aircraft& a, double aug, const Atmos& at, double mach,
+                            const double* __restrict__ T, double& burn) {
   const F16Br2 bm = F16_BR2(F16M_TG_ENG_IDLE_R, mach);
   const F16Br2 bd = F16_BR2(F16M_TG_ENG_IDLE_C, at.densalt);
   const F16Br2 bm2 = F16_BR2(F16M_TG_ENG_MIL_R, mach);
@@ -575,6 +598,12 @@ F16_HD double engine(Aircraft& a, double c_thr, const Atmos& at, double mach,
   }
   burn = a.ff * (kDt / 3600.0);
   return thrust;
+}
+
+F16_HD double engine(Aircraft& a, double c_thr, const Atmos& at, double mach,
+                     const double* __restrict__ T, double& burn) {
+  const double aug = engine_spool(a, c_thr, at);
+  return engine_thrust(a, aug, at, mach, T, burn);
 }
 
 // ---- aerodynamics (jsb_aero.py:75-107): 40 coefficient functions ----
@@ -621,35 +650,51 @@ F16_HD void gravity(const Kin& k, double gi[3]) {
 // ---- accelerations (jsb_accel.py:10-31) ----
 struct Accel { double ai[3], wdi[3], pba[3], ppq[3]; };   // vUVWidot, vPQRidot, vBodyAccel, vPQRi
 
-F16_HD void accelerations(const double B[3][3], const double wpqr[3], const Mass& mb,
-                          const double F[3], const double M[3], const double gi[3], Accel& o) {
-  double wq[3];   // vPQRi re-formed from vPQR, as the reference's accelerations do
+// What needs no force: vPQRi re-formed from vPQR (as the reference's accelerations do), the
+// gyroscopic moment c = wq x (J wq), and the reciprocal mass.
+struct AccelPre { double wq[3], c[3], sm; };
+F16_HD void accel_pre(const double B[3][3], const double wpqr[3], const double J[6], double mass,
+                      AccelPre& o) {
+  double* wq = o.wq;
 #pragma unroll
   for (int i = 0; i < 3; ++i) wq[i] = wpqr[i] + B[i][2] * kRot;
-  const double* J = mb.J;
   const double Jw0 = J[0] * wq[0] + J[3] * wq[1] + J[4] * wq[2];
   const double Jw1 = J[3] * wq[0] + J[1] * wq[1] + J[5] * wq[2];
   const double Jw2 = J[4] * wq[0] + J[5] * wq[1] + J[2] * wq[2];
-  const double m0 = M[0] - (wq[1] * Jw2 - wq[2] * Jw1);
-  const double m1 = M[1] - (wq[2] * Jw0 - wq[0] * Jw2);
-  const double m2 = M[2] - (wq[0] * Jw1 - wq[1] * Jw0);
-  const double* Ji = mb.Jinv;
+  o.c[0] = wq[1] * Jw2 - wq[2] * Jw1;
+  o.c[1] = wq[2] * Jw0 - wq[0] * Jw2;
+  o.c[2] = wq[0] * Jw1 - wq[1] * Jw0;
+  o.sm = fm_rcp(mass);
+}
+
+F16_HD void accel_post(const double B[3][3], const AccelPre& pre, const double Ji[6],
+                       const double F[3], const double M[3], const double gi[3], Accel& o) {
+  const double m0 = M[0] - pre.c[0], m1 = M[1] - pre.c[1], m2 = M[2] - pre.c[2];
   o.wdi[0] = Ji[0] * m0 + Ji[3] * m1 + Ji[4] * m2;
   o.wdi[1] = Ji[3] * m0 + Ji[1] * m1 + Ji[5] * m2;
   o.wdi[2] = Ji[4] * m0 + Ji[5] * m1 + Ji[2] * m2;
-  const double sm = fm_rcp(mb.mass);
 #pragma unroll
-  for (int i = 0; i < 3; ++i) o.pba[i] = F[i] * sm;
+  for (int i = 0; i < 3; ++i) o.pba[i] = F[i] * pre.sm;
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     o.ai[i] = (B[0][i] * o.pba[0] + B[1][i] * o.pba[1] + B[2][i] * o.pba[2]) + gi[i];
-    o.ppq[i] = wq[i];
+    o.ppq[i] = pre.wq[i];
   }
+}
+
+F16_HD void accelerations(const double B[3][3], const double wpqr[3], const Mass& mb,
+                          const double F[3], const double M[3], const double gi[3], Accel& o) {
+  AccelPre pre;
+  accel_pre(B, wpqr, mb.J, mb.mass, pre);
+  accel_post(B, pre, mb.Jinv, F, M, gi, o);
 }
 
 // ---- propagate: quaternion rect-Euler + normalize, vPQRi rect-Euler, ECI position AB3 on the
 // velocity history, ECI velocity AB2 on the acceleration history, Earth position angle ----
-F16_HD void propagate(Aircraft& a) {
+// The attitude, position and Earth angle need only the previous substep's quaternion rate and
+// velocities (propagate_pose, before the velocity histories shift); the rates and the velocity
+// need its accelerations (propagate_motion).
+F16_HD void propagate_pose(Aircraft& a) {
   {
     double q0 = a.q[0] + kDt * a.qd[0], q1 = a.q[1] + kDt * a.qd[1];
     double q2 = a.q[2] + kDt * a.qd[2], q3 = a.q[3] + kDt * a.qd[3];
@@ -661,16 +706,26 @@ F16_HD void propagate(Aircraft& a) {
     a.q[0] = q0; a.q[1] = q1; a.q[2] = q2; a.q[3] = q3;
   }
 #pragma unroll
+  for (int i = 0; i < 3; ++i)
+    a.p[i] = a.p[i] + (kDt / 12.0) * (23.0 * a.v[i] - 16.0 * a.vh1[i] + 5.0 * a.vh2[i]);
+  a.epa += kRot * kDt;
+}
+
+F16_HD void propagate_motion(Aircraft& a) {
+#pragma unroll
   for (int i = 0; i < 3; ++i) {
     a.wi[i] = a.wi[i] + kDt * a.wdi[i];
     const double v0 = a.v[i];
-    a.p[i] = a.p[i] + (kDt / 12.0) * (23.0 * v0 - 16.0 * a.vh1[i] + 5.0 * a.vh2[i]);
     a.v[i] = v0 + kDt * (1.5 * a.ai[i] - 0.5 * a.ah1[i]);
     a.vh2[i] = a.vh1[i];
     a.vh1[i] = v0;
     a.ah1[i] = a.ai[i];
   }
-  a.epa += kRot * kDt;
+}
+
+F16_HD void propagate(Aircraft& a) {
+  propagate_pose(a);
+  propagate_motion(a);
 }
 
 // Quaternion derivative for the next step (quat_qdot, jsb_frames.py:170-176).

@@ -11,22 +11,37 @@ namespace f16 {
 
 static __constant__ double c_image[F16M_IMAGE_LEN] = F16M_IMAGE_INIT;
 
-// Copy the model image into LDS: every load of a thread is issued before its first store, so
-// the copy costs one memory latency rather than one per element.  NT = threads per block.
+// The model image's copy into LDS, NT threads per block: every load of a thread is issued (load)
+// before its first store (store), so the copy costs one memory latency rather than one per
+// element, and a caller can issue other loads in between.  A barrier separates the stores from
+// the first read.
+template <int NT>
+struct ImageCopy {
+  static constexpr int kPer = (F16M_IMAGE_LEN + NT - 1) / NT;
+  double* T;
+  double v[kPer];
+  __device__ __forceinline__ void load(double* image) {
+    T = image;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const int i = threadIdx.x + j * NT;
+      v[j] = i < F16M_IMAGE_LEN ? c_image[i] : 0.0;
+    }
+  }
+  __device__ __forceinline__ void store() const {
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const int i = threadIdx.x + j * NT;
+      if (i < F16M_IMAGE_LEN) T[i] = v[j];
+    }
+  }
+};
+
 template <int NT>
 __device__ __forceinline__ void stage_image(double* T) {
-  constexpr int kPer = (F16M_IMAGE_LEN + NT - 1) / NT;
-  double v[kPer];
-#pragma unroll
-  for (int j = 0; j < kPer; ++j) {
-    const int i = threadIdx.x + j * NT;
-    v[j] = i < F16M_IMAGE_LEN ? c_image[i] : 0.0;
-  }
-#pragma unroll
-  for (int j = 0; j < kPer; ++j) {
-    const int i = threadIdx.x + j * NT;
-    if (i < F16M_IMAGE_LEN) T[i] = v[j];
-  }
+  ImageCopy<NT> c;
+  c.load(T);
+  c.store();
   __syncthreads();
 }
 

@@ -1070,12 +1070,12 @@ __device__ __forceinline__ void norm_partials_from_tiles(const float* S_all, dou
 // finished engagements are rebuilt from their autoreset state by the advance role after the
 // flush, as the single-wave kernel's terminal path does; without terminal_obs their first
 // build is not stored.  Results equal env_post_step_kernel's bit for bit.
-template <int D, bool FULL>
+template <int D, bool FULL, int NG = kPostGroups>
 struct PostSplitLds {
-  float S_all[kPostGroups][kRowBlock * tile_pitch<D, FULL>()];
-  uint64_t sh_mask[kPostGroups][3];    // live, finished and pool-table finished rows
-  long sh_pick[kPostGroups][kRowBlock];  // pool table row of each pool-table autoreset
-  double sh_norm[FULL ? 8 * D : 1];      // RunningNorm partials per phase (full tile)
+  float S_all[NG][kRowBlock * tile_pitch<D, FULL>()];
+  uint64_t sh_mask[NG][3];             // live, finished and pool-table finished rows
+  long sh_pick[NG][kRowBlock];         // pool table row of each pool-table autoreset
+  double sh_norm[FULL && NG == 2 ? 8 * D : 1];   // RunningNorm partials per phase (full tile)
 };
 
 template <int D, bool FULL>
@@ -1290,10 +1290,12 @@ __global__ __launch_bounds__(kPostSplitBlock) void env_post_step_split_kernel(
 // bit for bit.
 constexpr int kQuadPostBlock = 4 * kRowBlock * kPostGroups;   // 512
 
-template <int D>
+// NG: 64-aircraft groups per workgroup; a launch with norm partials has two (128 rows are one
+// norm block).
+template <int D, int NG = kPostGroups>
 __device__ __forceinline__ void post_quad_body(const F16EnvStepIO& io, const F16Recon& r,
                                                const F16RewardCfg& c, const Origin& O,
-                                               PostSplitLds<D, true>& L) {
+                                               PostSplitLds<D, true, NG>& L) {
   auto& S_all = L.S_all;
   auto& sh_mask = L.sh_mask;
   auto& sh_pick = L.sh_pick;
@@ -1305,7 +1307,7 @@ __device__ __forceinline__ void post_quad_body(const F16EnvStepIO& io, const F16
   const int role = grp == 0 ? (wave & 3) : 3 - (wave & 3);
   const int gtid = (int)(threadIdx.x & (NTG - 1));
   float* const S = S_all[grp];
-  const long a0 = ((long)blockIdx.x * kPostGroups + grp) * kRowBlock, a = a0 + lane;
+  const long a0 = ((long)blockIdx.x * NG + grp) * kRowBlock, a = a0 + lane;
   const long nac = 2L * r.nenv;
   const int n = (int)max(0L, min((long)kRowBlock, nac - a0));
   const bool on = a < nac;                              // nac is even: pairs agree
@@ -1426,9 +1428,9 @@ __device__ __forceinline__ void post_quad_body(const F16EnvStepIO& io, const F16
     flush_tile<D, true, NTG>(S, a0, n, live, io.obs, 0, nullptr, gtid);
   bool any_fresh = false;   // uniform over the workgroup, so every thread meets the same barriers
 #pragma unroll
-  for (int q = 0; q < kPostGroups; ++q) any_fresh |= sh_mask[q][1] != 0;
+  for (int q = 0; q < NG; ++q) any_fresh |= sh_mask[q][1] != 0;
   if (!any_fresh) {
-    if (io.norm_partial)
+    if (NG == 2 && io.norm_partial)
       norm_partials_from_tiles<D, kQuadPostBlock>(&S_all[0][0], sh_norm,
                                                   (long)blockIdx.x * 2 * kRowBlock, nac,
                                                   blockIdx.x, io, threadIdx.x);
@@ -1470,7 +1472,7 @@ __device__ __forceinline__ void post_quad_body(const F16EnvStepIO& io, const F16
   flush_sparse<D, true, NTG>(S, a0, fresh & ~from_table, io.obs, gtid);
   if (from_table)
     copy_pool_rows<D, true, NTG>(S, a0, from_table, sh_pick[grp], io, io.pool_obs, io.obs, gtid);
-  if (io.norm_partial) {
+  if (NG == 2 && io.norm_partial) {
     __syncthreads();     // (workgroup-uniform) the copied rows have landed in the tiles
     norm_partials_from_tiles<D, kQuadPostBlock>(&S_all[0][0], sh_norm,
                                                 (long)blockIdx.x * 2 * kRowBlock, nac,
@@ -1540,51 +1542,69 @@ __global__ __launch_bounds__(kPostSplitBlock) void env_step_fused_kernel(
   post_split_body<D, true>(io, r, c, O, L.post);
 }
 
-// The same step on 512-thread workgroups: each 64 aircraft on four wavefronts in both phases
-// (fdm_quad.h's four physics roles, then post_quad_body's four post-physics roles), so that at
+// The same step with each 64 aircraft on four wavefronts in both phases (fdm_quad.h's four physics
+// roles, then post_quad_body's four post-physics roles).  NG = 2 (512-thread workgroups): at
 // 16,384 engagements every SIMD holds two wavefronts instead of one.  Results equal
 // env_step_fused_kernel's bit for bit.
-template <int D>
+template <int D, int NG>
 union EnvQuadLds {
   struct {
     double T[F16M_IMAGE_LEN];
-    f16::QuadX X[f16::kQuadGroups];
+    f16::QuadX X[NG];
   } fdm;
-  PostSplitLds<D, true> post;
+  PostSplitLds<D, true, NG> post;
 };
 static_assert(f16::kQuadBlock == kQuadPostBlock && f16::kQuadAircraft == kPostGroups * kRowBlock,
               "the four-role physics groups and post-physics groups must cover the same aircraft");
 
-template <int FCS_RATE, int D>
-__global__ __launch_bounds__(kQuadPostBlock) void env_step_quad_kernel(
-    const double* __restrict__ act, int S, double* act_keep,
-    unsigned char* state_finite, const F16EnvStepIO io, F16Recon r, F16RewardCfg c,
-    Origin O) {
-  __shared__ EnvQuadLds<D> L;
-  f16::stage_image<kQuadPostBlock>(L.fdm.T);
+struct EnvStepArgs {
+  const double* act;
+  int S;
+  double* act_keep;
+  unsigned char* state_finite;
+  F16EnvStepIO io;
+  F16Recon r;
+  F16RewardCfg c;
+  Origin O;
+};
+
+template <int FCS_RATE, int D, int NG>
+__global__ __launch_bounds__(256 * NG) void env_step_quad_kernel(const EnvStepArgs A) {
+  __shared__ EnvQuadLds<D, NG> L;
+  f16::ImageCopy<256 * NG> image;   // stored by the roles once their state loads are issued
+  image.load(L.fdm.T);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int grp = wave >> 2;
-  const int role = f16::quad_role(grp, wave & 3);
-  const int nac = 2 * r.nenv;
-  const int i = blockIdx.x * f16::kQuadAircraft + grp * 64 + lane;
+  const int role = f16::quad_role(NG == 1 ? (int)(blockIdx.x & 1) : grp, wave & 3);
+  const int nac = 2 * A.r.nenv;
+  const int i = blockIdx.x * (64 * NG) + grp * 64 + lane;
   const bool store = i < nac;
   const int ia = store ? i : nac - 1;   // lanes past the batch shadow the last aircraft
-  double* const st = io.states + ia;
-  // (two groups per workgroup: the physics roles run with their phase priorities, fdm_quad.h)
+  double* const st = A.io.states + ia;
+  const long ld = A.io.ld;
+  const int S = A.S;
+  constexpr bool kPrio = NG == 2;   // two waves per SIMD to arbitrate between (fdm_quad.h)
   if (role == f16::kRoleKin)
-    f16::quad_kin<FCS_RATE, true>(st, io.ld, S, store, nullptr, 0, L.fdm.T, L.fdm.X[grp], lane,
-                                  true);
+    f16::quad_kin<FCS_RATE, kPrio>(image, st, ld, S, store, nullptr, 0, L.fdm.T, L.fdm.X[grp],
+                                   lane, true);
   else if (role == f16::kRoleAero)
-    f16::quad_aero<FCS_RATE, true>(S, L.fdm.T, L.fdm.X[grp], lane, true);
+    f16::quad_aero<FCS_RATE, kPrio>(image, S, L.fdm.T, L.fdm.X[grp], lane, true);
   else if (role == f16::kRoleFcs)
-    f16::quad_fcs<FCS_RATE, true>(st, io.ld, act + 4L * ia, S, store, L.fdm.T, L.fdm.X[grp],
-                                  lane, true, act_keep ? act_keep + 4L * ia : nullptr);
+    f16::quad_fcs<FCS_RATE, kPrio>(image, st, ld, A.act + 4L * ia, S, store, L.fdm.T, L.fdm.X[grp],
+                                   lane, true, A.act_keep ? A.act_keep + 4L * ia : nullptr);
   else
-    f16::quad_air<FCS_RATE, true>(st, io.ld, act + 4L * ia, S, store, L.fdm.T, L.fdm.X[grp],
-                                  lane, state_finite + ia);
+    f16::quad_air<FCS_RATE, kPrio>(image, st, ld, A.act + 4L * ia, S, store, L.fdm.T, L.fdm.X[grp],
+                                   lane, A.state_finite + ia);
   __syncthreads();   // the new states, finite flags and actions are written; LDS is free
-  post_quad_body<D>(io, r, c, O, L.post);
+  // The post-physics arguments are read here through a pointer the compiler cannot see through:
+  // read above the substep loop (they are launch constants) they took the scalar registers the
+  // loop's constants need.
+  typedef const EnvStepArgs __attribute__((address_space(4)))* ArgsPtr;
+  ArgsPtr P = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(P));
+  const EnvStepArgs& B = *(const EnvStepArgs*)P;
+  post_quad_body<D, NG>(B.io, B.r, B.c, B.O, L.post);
 }
 
 // Masked autoreset without a step: engagements with mask[e] != 0 get an initial-condition pool
@@ -1655,19 +1675,27 @@ static bool rows_aligned(const float* p, int obs_dim) {
   return ((uintptr_t)p & (obs_dim % 4 == 0 ? 15u : 7u)) == 0;
 }
 
+// Compute units and LDS per compute unit of the device (asked once).
+struct DeviceSize { int cus = 0, lds = 0; };
+static const DeviceSize& resident_device() {
+  static const DeviceSize d = [] {
+    DeviceSize q;
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&q.cus, hipDeviceAttributeMultiprocessorCount, dev);
+    (void)hipDeviceGetAttribute(&q.lds, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev);
+    if (q.cus <= 0) q.cus = 256;
+    if (q.lds <= 0) q.lds = 160 * 1024;
+    return q;
+  }();
+  return d;
+}
+
 // Whether a row launch over nenv engagements keeps every workgroup resident at once with the
 // full-row tile (limited by LDS per CU); otherwise the vector-block tile is used, which lets
 // four wavefronts share a CU.  `groups`: 64-row tiles per workgroup.
 static bool full_tile_resident(int nenv, int obs_dim, int groups = 1) {
-  static int cus = 0, lds = 0;
-  if (cus == 0) {
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    (void)hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev);
-    if (cus <= 0) cus = 256;
-    if (lds <= 0) lds = 160 * 1024;
-  }
+  const int cus = resident_device().cus, lds = resident_device().lds;
   const long rows = (long)kRowBlock * groups;
   const long blocks = (2L * nenv + rows - 1) / rows;
   const long tile = rows * (obs_dim | 1) * (long)sizeof(float);
@@ -1831,12 +1859,12 @@ static int env_step(const F16EnvStepIO* io, const F16Recon* rec, const F16Reward
     return post_step_launch(&x, rec, cfg, stream, true, false);
   }
   hipStream_t s = (hipStream_t)stream;
+  const EnvStepArgs args{act, substeps, keep, state_finite, x, *rec, *cfg, origin()};
 #define F16_ENV_STEP(R, D)                                                                      \
   do {                                                                                          \
     if (quad)                                                                                   \
-      hipLaunchKernelGGL((env_step_quad_kernel<R, D>), grid_groups(rec->nenv),                  \
-                         dim3(kQuadPostBlock), 0, s, act, substeps, keep, state_finite, x, *rec,\
-                         *cfg, origin());                                                       \
+      hipLaunchKernelGGL((env_step_quad_kernel<R, D, 2>), grid_groups(rec->nenv),               \
+                         dim3(kQuadPostBlock), 0, s, args);                                     \
     else                                                                                        \
       hipLaunchKernelGGL((env_step_fused_kernel<R, D>), grid_groups(rec->nenv),                 \
                          dim3(kPostSplitBlock), 0, s, act, substeps, keep, state_finite, x,     \

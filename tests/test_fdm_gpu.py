@@ -322,6 +322,33 @@ def test_split_kernel_equals_onelane(gpu, rate, nenv, S, pad):
         assert torch.equal(sa[:, :nac], sim._state_soa)
 
 
+@pytest.mark.parametrize("nenv,S", [(65, 1), (65, 2), (130, 6), (16400, 6)])
+def test_quad_kernel_equals_onelane_through_mach_one(gpu, nenv, S):
+    """Aircraft on both sides of Mach 1 in every wavefront: between substeps the four-wave kernel
+    leaves the calibrated airspeed's supersonic passes out (the FCS channels only test it against
+    250 kt and less) and makes them on the last; every stored value equals the one-lane kernel's
+    bit for bit over 10 decisions of S substeps, with one and two groups per workgroup."""
+    icm = import_pkg("ic")
+    L = import_pkg("_lib")
+    nac = 2 * nenv
+    rows = icm.sample_tailchase(nenv, seed=11)
+    rows[:, 3] = np.random.default_rng(11).uniform(750.0, 1500.0, nac)        # ft/s
+    sim = _sim(nenv, 60, S)
+    sim.seed_rows(torch.as_tensor(rows, device=gpu))
+    a = sim._state_soa.clone()
+    b = a.clone()
+    acts = icm.random_bin_actions(10, nac, seed=11)
+    for d in range(10):
+        at = torch.as_tensor(acts[d], device=gpu).contiguous()
+        for fn, st in ((L.lib().f16_fdm_step_batch, a), (L.lib().f16_fdm_step_batch_onelane, b)):
+            L.check(fn(L.ptr(st), nac, L.ptr(at), nac, S, 60, None, nac, L.stream_handle(gpu)),
+                    "step")
+        same = a.view(torch.int64) == b.view(torch.int64)
+        assert bool(same.all()), (d, torch.nonzero(~same)[:4])
+    mach = a[74]                                       # previous-frame Mach number
+    assert bool((mach > 1.0).any()) and bool((mach < 1.0).any())
+
+
 def test_nonfinite_lane_is_isolated(gpu):
     g = oracle_lib.golden("seed_golden.npz")
     sim = _sim(4)
