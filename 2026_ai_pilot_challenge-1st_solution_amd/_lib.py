@@ -118,6 +118,7 @@ _SIGNATURES = {
     "f16_env_step": (_i, [ctypes.POINTER(F16EnvStepIO), _RP, _CP, _vp, _i, _i, _vp, _vp]),
     "f16_env_step_tworole": (_i, [ctypes.POINTER(F16EnvStepIO), _RP, _CP, _vp, _i, _i, _vp, _vp]),
     "f16_env_post_step_norm_fusable": (_i, [_i, _i]),
+    "f16_env_step_norm_pays": (_i, [_i, _i]),
     "f16_env_reseed": (_i, [ctypes.POINTER(F16EnvStepIO), _RP, _vp, _vp]),
     "f16_state9": (_i, [_vp, _l, _i, _vp, _vp]),
     "f16_future_labels": (_i, [_vp, _vp, _i, _i, _d, _vp, _vp, _vp]),

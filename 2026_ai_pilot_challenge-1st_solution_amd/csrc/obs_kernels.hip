@@ -1544,8 +1544,8 @@ __global__ __launch_bounds__(kPostSplitBlock) void env_step_fused_kernel(
 
 // The same step with each 64 aircraft on four wavefronts in both phases (fdm_quad.h's four physics
 // roles, then post_quad_body's four post-physics roles).  NG = 2 (512-thread workgroups): at
-// 16,384 engagements every SIMD holds two wavefronts instead of one.  Results equal
-// env_step_fused_kernel's bit for bit.
+// 16,384 engagements every SIMD holds two wavefronts instead of one.  NG = 1: a small batch
+// spreads over twice the CUs, one wavefront per SIMD, so neither phase shares its issue slots.  Results equal env_step_fused_kernel's bit for bit.
 template <int D, int NG>
 union EnvQuadLds {
   struct {
@@ -1700,6 +1700,15 @@ static bool full_tile_resident(int nenv, int obs_dim, int groups = 1) {
   const long blocks = (2L * nenv + rows - 1) / rows;
   const long tile = rows * (obs_dim | 1) * (long)sizeof(float);
   return blocks <= (long)(lds / tile) * cus;
+}
+
+// Whether the one-launch step takes one 64-aircraft group per workgroup: while every such
+// workgroup has a CU of its own (8,192 engagements on 256 CUs).  Rollout of 64 steps at 200 /
+// 4,000 / 9,000 / 15,000 engagements with two groups per workgroup and with one: 4.34 / 4.78 /
+// 5.69 / 5.91 ms and 3.97 / 4.43 / 5.64 / 6.14 ms, the latter with the norm's partial sums in a
+// launch of their own; a league of 2,000 and 12,000 (32 steps): 6.15, 3.39 and 5.63, 3.42 ms.
+static bool env_step_one_group(int nenv) {
+  return 2L * nenv <= (long)kRowBlock * resident_device().cus;
 }
 
 static int check_cfg(const F16RewardCfg* c) {
@@ -1860,11 +1869,16 @@ static int env_step(const F16EnvStepIO* io, const F16Recon* rec, const F16Reward
   }
   hipStream_t s = (hipStream_t)stream;
   const EnvStepArgs args{act, substeps, keep, state_finite, x, *rec, *cfg, origin()};
+  // (a launch that forms norm partials, blocks of 128 rows, has two groups)
+  const bool two = x.norm_partial || !env_step_one_group(rec->nenv);
 #define F16_ENV_STEP(R, D)                                                                      \
   do {                                                                                          \
-    if (quad)                                                                                   \
+    if (quad && two)                                                                            \
       hipLaunchKernelGGL((env_step_quad_kernel<R, D, 2>), grid_groups(rec->nenv),               \
                          dim3(kQuadPostBlock), 0, s, args);                                     \
+    else if (quad)                                                                              \
+      hipLaunchKernelGGL((env_step_quad_kernel<R, D, 1>), grid_rows(rec->nenv),                 \
+                         dim3(kQuadPostBlock / 2), 0, s, args);                                 \
     else                                                                                        \
       hipLaunchKernelGGL((env_step_fused_kernel<R, D>), grid_groups(rec->nenv),                 \
                          dim3(kPostSplitBlock), 0, s, act, substeps, keep, state_finite, x,     \
@@ -1894,6 +1908,10 @@ extern "C" int f16_env_step_tworole(const F16EnvStepIO* io, const F16Recon* rec,
 extern "C" int f16_env_post_step_norm_fusable(int nenv, int obs_dim) {
   if (nenv < 1 || (obs_dim != 184 && obs_dim != 214)) return 0;
   return full_tile_resident(nenv, obs_dim, kPostGroups) ? 1 : 0;
+}
+
+extern "C" int f16_env_step_norm_pays(int nenv, int obs_dim) {
+  return f16_env_post_step_norm_fusable(nenv, obs_dim) && !env_step_one_group(nenv) ? 1 : 0;
 }
 
 extern "C" int f16_env_post_step_onewave(const F16EnvStepIO* io, const F16Recon* rec,

@@ -199,6 +199,7 @@ class SelfPlayRollout:
         env, T = self.env, self.T
         dev = self.device
         g0 = 0 if pol_base is not None else self.global_step
+        fuse_norm = self.fuse_norm and env.norm_fuse_pays()
         self.finite_acc.fill_(1)
         self.b_done[0].copy_(self.next_done)
         if self.want_stats:
@@ -209,14 +210,14 @@ class SelfPlayRollout:
             if self.b_aux_features is not None:       # features of s_t (ppo_gpu.py:1876-1879)
                 self.b_aux_features[t].copy_(env.obr.aux_features)
             if self.update_norm:
-                if self.fuse_norm and t > 0:
+                if fuse_norm and t > 0:
                     self.norm.merge(self.nac)     # partials from step t - 1's post-physics launch
                 else:
                     self.norm.update(obs)
             self._policy(obs, g0 + t, pol_base, nobs_out=self.b_obs[t], act_idx=self.b_act[t],
                          logp=self.b_logp[t], value=self.b_val[t], env_actions=env.sim.actions)
             done_t = self.b_done[t + 1] if t + 1 < T else self.next_done
-            fused = self.norm if (self.fuse_norm and t + 1 < T) else None
+            fused = self.norm if (fuse_norm and t + 1 < T) else None
             self.next_obs = env.step_rollout(self.b_rew[t], done_t, self.finite_acc,
                                              step_base=env_base, step=t, norm=fused)
             if self.want_stats:

@@ -447,6 +447,13 @@ class GpuDogfightVecEnv:
         """Whether step_rollout can also form the RunningNorm partial sums of its new rows."""
         return bool(self.obr._lib.f16_env_post_step_norm_fusable(self.nenv, self.OBS_SIZE))
 
+    def norm_fuse_pays(self):
+        """Whether a rollout's step is faster with the norm partials formed in its launch than
+        with a separate RunningNorm.update: in a batch that gives 64-aircraft workgroups a compute
+        unit each the one-launch step uses those, which cannot form the 128-row partials."""
+        return not self.fused_step or bool(
+            self.obr._lib.f16_env_step_norm_pays(self.nenv, self.OBS_SIZE))
+
     def step_rollout(self, reward_f32, done_f32, finite_acc, step_base=None, step=0, norm=None,
                      reward0_f32=None, terminal_hp=None, terminal_alt_m=None):
         """The rollout collector's step: the controls already sit in sim.actions (written by the

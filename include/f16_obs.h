@@ -152,7 +152,8 @@ typedef struct F16EnvStepIO {
  * workgroup of the post-physics step's full-row tile is resident at once (as
  * f16_env_post_step_norm_fusable reports), one launch does both: each 512-thread workgroup runs
  * the physics of its 128 aircraft on four wavefronts per 64 aircraft, then their post-physics
- * step, again on four (two wavefronts per SIMD at 16,384 engagements); otherwise the two launches
+ * step, again on four (two wavefronts per SIMD at 16,384 engagements; 256 threads and 64 aircraft
+ * while such workgroups have a compute unit each); otherwise the two launches
  * are issued.  Results equal the two entry points' bit for bit.  Every argument is checked before
  * anything is launched. */
 int f16_env_step(const F16EnvStepIO *io, const F16Recon *rec, const F16RewardCfg *cfg,
@@ -185,6 +186,11 @@ int f16_env_post_step(const F16EnvStepIO *io, const F16Recon *rec, const F16Rewa
  * of its new observation rows (io->norm_partial): every row's block sits whole in one
  * workgroup's staging tile.  0 otherwise (the caller then runs f16_norm_update). */
 int f16_env_post_step_norm_fusable(int nenv, int obs_dim);
+
+/* 1 when it is also the faster way for f16_env_step: while 64-aircraft workgroups have a
+ * compute unit each, the one launch takes 64 aircraft per workgroup and the partials (128-row
+ * blocks) would hold it to 128. */
+int f16_env_step_norm_pays(int nenv, int obs_dim);
 
 /* The same step with one wavefront per 64 aircraft (f16_env_post_step spreads each group's
  * row build over four wavefronts -- advance, scalar block, vector-block frames 0-2 and 3-5 --

@@ -656,6 +656,45 @@ def test_env_step_one_launch_equals_two(gpu, obs_dim, nenv, fcs, roles):
         assert float(norms[0].count) > 1.0
 
 
+@pytest.mark.parametrize("obs_dim,nenv", [(184, 33), (214, 777), (184, 8192), (184, 8193)])
+def test_env_step_group_count_edges(gpu, obs_dim, nenv):
+    """The one launch takes 64 aircraft per workgroup while each has a compute unit (8,192
+    engagements on 256) and 128 beyond: on both sides of that size, and with ragged last groups,
+    step and step_rollout equal the two launches bit for bit over steps with autoresets."""
+    E = import_pkg("rl_env").GpuDogfightVecEnv
+    envs = [E(nenv, seed=21, ic_pool_size=32, obs_dim=obs_dim, max_engage_time_s=0.6)
+            for _ in range(2)]
+    envs[1].fused_step = False
+    for env in envs:
+        env.enable_aux_capture()
+        env.reset(stagger=True, max_stagger_steps=6)
+    rng = np.random.default_rng(21)
+    bits = lambda t: t.contiguous().view(torch.int32 if t.element_size() == 4 else
+                                         torch.int64 if t.element_size() == 8 else torch.uint8)
+    same = lambda x, y: torch.equal(bits(x), bits(y))
+    resets = 0
+    for k in range(8):
+        act = torch.as_tensor(rng.uniform(-1, 1, (2 * nenv, 4)), device=gpu)
+        outs = []
+        for env in envs:
+            if k % 2 == 0:
+                o, r, d, i = env.step(act)
+                outs.append([o, r, d, i["terminal_obs"], i["terminal_hp"],
+                             i["terminal_state_finite"]])
+                resets += int(d.sum())
+            else:
+                env.sim.actions.copy_(act)
+                rew = torch.zeros(2 * nenv, dtype=torch.float32, device=gpu)
+                dn = torch.zeros(nenv, dtype=torch.float32, device=gpu)
+                fa = torch.ones(nenv, dtype=torch.uint8, device=gpu)
+                outs.append([env.step_rollout(rew, dn, fa), rew, dn, fa])
+        assert all(same(x, y) for x, y in zip(*outs)), k
+        assert same(envs[0].sim._state_soa, envs[1].sim._state_soa), k
+        for name in ("hp", "t_sec", "aux_features", "_hist_soa", "_att_soa", "_pqr_soa"):
+            assert same(getattr(envs[0].obr, name), getattr(envs[1].obr, name)), (k, name)
+    assert resets > 0
+
+
 def test_step_training_and_capture_switch(gpu):
     """The root lineage's surface (cuda_fdm/rl_env.py:518-529): step_training and
     step(capture_terminal_obs=False) return the same observation, reward, done and info as a
