@@ -10,6 +10,7 @@ stream with no synchronisation; data readiness across streams is the caller's (w
 the tensors a launch touches are marked with `record` so their memory outlives the launch.
 """
 import ctypes
+import operator
 import os
 
 import torch  # noqa: F401  (loads the HIP runtime the library binds to)
@@ -187,11 +188,32 @@ def stream_handle(device=None):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
+class _LaunchStream:
+    """The caller's current stream on a device, by its raw handle; the torch.cuda.Stream object is
+    made only where a tensor has to be recorded (building one costs more than a launch)."""
+    __slots__ = ("cuda_stream", "index")
+
+    def __init__(self, cuda_stream, index):
+        self.cuda_stream, self.index = cuda_stream, index
+
+    def torch_stream(self):
+        s = torch.cuda.current_stream(self.index)
+        if s.cuda_stream != self.cuda_stream:
+            raise RuntimeError("the current stream changed between a launch and its record")
+        return s
+
+
 def launch_stream(device=None):
     """(stream, C handle) of the caller's current stream on `device`: every launch of this
     library goes there, and `record` marks its tensors as used on the same stream."""
-    s = torch.cuda.current_stream(device)
-    return s, ctypes.c_void_p(s.cuda_stream)
+    index = device.index if isinstance(device, torch.device) else None
+    if index is None:
+        if device is not None and not isinstance(device, torch.device):
+            index = torch.device(device).index
+        if index is None:
+            index = torch.cuda.current_device()
+    h = torch._C._cuda_getCurrentRawStream(index)
+    return _LaunchStream(h, index), ctypes.c_void_p(h)
 
 
 def record(stream, tensors):
@@ -216,6 +238,8 @@ def record(stream, tensors):
             t._f16_streams = seen
         elif tag in seen:
             continue
+        if isinstance(stream, _LaunchStream):
+            stream = stream.torch_stream()
         t.record_stream(stream)
         seen.add(tag)
 
@@ -229,7 +253,7 @@ def record_owned(owner, stream, tensors):
     prev = owner.__dict__.get("_f16_owned")
     key = stream.cuda_stream
     if (prev is not None and prev[0] == key and len(prev[1]) == len(tensors)
-            and all(a is b for a, b in zip(prev[1], tensors))):
+            and all(map(operator.is_, prev[1], tensors))):
         return
     record(stream, tensors)
     owner._f16_owned = (key, tensors)

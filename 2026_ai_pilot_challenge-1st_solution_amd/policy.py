@@ -269,20 +269,21 @@ class PolicyStep:
             nphys = nlog
         if obs.shape[0] < nphys:
             raise ValueError("obs has fewer rows than the rows addressed")
-        for t, rows_needed, w in ((nobs_out, nlog, self.obs_dim), (act_idx, nlog, 4),
-                                  (logp, nlog, 1), (value, nlog, 1), (env_actions, nphys, 4),
-                                  (logits_out, nlog, 84)):
+        f32 = torch.float32
+        for t, rows_needed, w, dtype in ((nobs_out, nlog, self.obs_dim, f32),
+                                         (act_idx, nlog, 4, torch.int64), (logp, nlog, 1, f32),
+                                         (value, nlog, 1, f32),
+                                         (env_actions, nphys, 4, torch.float64),
+                                         (logits_out, nlog, 84, f32)):
             if t is None:
                 continue
-            if not t.is_contiguous() and t is not nobs_out:
+            if t is not nobs_out and not t.is_contiguous():
                 raise ValueError("output buffers must be contiguous")
-            if t.shape[0] < rows_needed or (t.dim() > 1 and t.shape[1] < w):
+            shape = t.shape
+            if shape[0] < rows_needed or (len(shape) > 1 and shape[1] < w):
                 raise ValueError("output buffer too small for the rows addressed")
-        dtypes = ((act_idx, torch.int64), (logp, torch.float32), (value, torch.float32),
-                  (env_actions, torch.float64), (logits_out, torch.float32),
-                  (nobs_out, torch.float32))
-        if any(t is not None and t.dtype != d for t, d in dtypes):
-            raise ValueError("output buffer dtype mismatch")
+            if t.dtype != dtype:
+                raise ValueError("output buffer dtype mismatch")
         a = _lib.F16PolicyArgs()
         a.obs, a.obs_ld, a.obs_dim = obs.data_ptr(), obs.stride(0), self.obs_dim
         if norm is not None:

@@ -35,13 +35,12 @@ def gae(rew, val, done, last_val, next_done, gamma=0.997, lam=0.95):
     rew, val, done, last_val, next_done = (f(x) for x in (rew, val, done, last_val, next_done))
     adv = torch.empty_like(rew)
     ret = torch.empty_like(rew)
-    # gamma*lambda is formed in double then rounded once, as the reference's Python scalars are
-    gl = float(torch.tensor(float(gamma) * float(lam), dtype=torch.float32))
-    g = float(torch.tensor(float(gamma), dtype=torch.float32))
+    # gamma*lambda is formed in double then rounded once (c_float), as the reference's Python
+    # scalars are
     stream, h = _lib.launch_stream(dev)
-    rc = _lib.lib().f16_gae(_lib.ptr(rew), _lib.ptr(val), _lib.ptr(done), _lib.ptr(last_val),
-                            _lib.ptr(next_done), T, nenv, nag, _lib.ctypes.c_float(g),
-                            _lib.ctypes.c_float(gl), _lib.ptr(adv), _lib.ptr(ret), h)
+    rc = _lib.lib().f16_gae(rew.data_ptr(), val.data_ptr(), done.data_ptr(), last_val.data_ptr(),
+                            next_done.data_ptr(), T, nenv, nag, float(gamma),
+                            float(gamma) * float(lam), adv.data_ptr(), ret.data_ptr(), h)
     _lib.record(stream, (rew, val, done, last_val, next_done))
     _lib.check(rc, "f16_gae")
     return adv, ret
