@@ -88,7 +88,7 @@ struct Work {
   float* fmid;          // [ceil(nwg / kColRows)][kPartCols] first level of the fpart sums
   float* wpart;         // [nchunk][nflat - 257]
   long ld;              // rows, rounded up to 64
-  int nwg, nchunk, chunk_rows, nadv;
+  int nwg, nchunk, chunk_rows, nadv, tile_rows;
   long bytes;
 };
 
@@ -99,7 +99,7 @@ struct Work {
 // 128-byte row segment its own DRAM page.  Within a block the feature stride is 64 elements.
 constexpr long kUBlock = 64;
 __host__ __device__ inline __bf16* ublock(__bf16* buf, long nf, long m0) {
-  return buf + (m0 / kUBlock) * nf * kUBlock;
+  return buf + (m0 / kUBlock) * nf * kUBlock + m0 % kUBlock;
 }
 
 constexpr int kColRows = 64;                     // rows per block of the two-level column sum
@@ -109,12 +109,14 @@ inline int norm_blocks(long n) { return (int)((n + kNormBlockElems - 1) / kNormB
 
 inline int wgrad_tiles(int kp) { return 2 * ((kp + 255) / 256) + 1 + 1 + 1; }
 
-inline Work layout(int obs_dim, long mb_rows, void* base, int wg_slots = kWgradSlots) {
+inline Work layout(int obs_dim, long mb_rows, void* base, int wg_slots = kWgradSlots,
+                   int tile_rows = 64) {
   Work w{};
   const int kp = (obs_dim + 31) / 32 * 32;
   const Flat F{obs_dim};
   w.ld = (mb_rows + 63) / 64 * 64;
-  w.nwg = (int)(w.ld / 64);
+  w.tile_rows = tile_rows;
+  w.nwg = (int)(w.ld / tile_rows);
   const int tiles = wgrad_tiles(kp);
   // chunks of 64-row stages: one workgroup per resident slot (a grid a little above a
   // multiple of the slots leaves a mostly idle last round), at least 4 stages each
@@ -139,10 +141,10 @@ inline Work layout(int obs_dim, long mb_rows, void* base, int wg_slots = kWgradS
   w.dh1t = reinterpret_cast<__bf16*>(take(512L * w.ld * 2));
   w.dh2t = reinterpret_cast<__bf16*>(take(512L * w.ld * 2));
   w.dzt = reinterpret_cast<__bf16*>(take((long)kLogitsPad * w.ld * 2));
-  w.fpart = reinterpret_cast<float*>(take((long)w.nwg * kPartCols * 4));
+  w.fpart = reinterpret_cast<float*>(take(w.ld / 32 * kPartCols * 4));
   w.nadv = (int)((w.ld + kAdvThreads * kAdvPer - 1) / (kAdvThreads * kAdvPer));
   w.advp = reinterpret_cast<double*>(take((long)w.nadv * 2 * sizeof(double)));
-  w.fmid = reinterpret_cast<float*>(take((long)kColGroups(w.nwg) * kPartCols * 4));
+  w.fmid = reinterpret_cast<float*>(take(kColGroups(w.ld / 32) * kPartCols * 4));
   w.wpart = reinterpret_cast<float*>(take(cap * (F.n() - 257) * 4));
   w.bytes = off;
   return w;
@@ -282,13 +284,13 @@ __device__ __forceinline__ float sum64(float x) {
 constexpr int kBufWord3 = 0x00020000;   // gfx9 buffer descriptor word 3 (raw, 32-bit data format)
 constexpr int kMaxMinibatchRows = 1 << 24;
 
-// LDS [row][pitch] bf16 tile of 64 rows x NF features (NF a multiple of 32) -> unit-major global
+// LDS [row][pitch] bf16 tile of 32 NR rows x NF features (NF a multiple of 32) -> unit-major global
 // dst[f][m0 + row], transposed by the matrix cores: D = A I over two 16-wide K slices, A the
 // tile's rows read as the usual activation operand (16-byte, bank-conflict-free) and I the
 // identity split over the slices, so result lane l holds feature l % 32 of rows
 // 32r + 8g + 4(l / 32) + 0..3 -- one 8-byte store per 4 rows.  Exact: each output is one
 // product x * 1 plus zero products.  Blocks of 32 features x 32 rows go round the waves.
-template <int NF>
+template <int NF, int NR>
 __device__ __forceinline__ void transpose_t(const __bf16* S, int pitch, __bf16* dst, long ld,
                                             long m0, int wave, int lane) {
   const int lr = lane & 31, kb = (lane >> 5) * 8;
@@ -301,8 +303,8 @@ __device__ __forceinline__ void transpose_t(const __bf16* S, int pitch, __bf16* 
   const __amdgpu_buffer_rsrc_t rs =
       __builtin_amdgcn_make_buffer_rsrc(dst + m0, 0, 0x7fffffff, kBufWord3);
   const int lo = 2 * (lr * (int)ld + (lane >> 5) * 4);
-  for (int blk = wave; blk < (NF / 32) * 2; blk += kWaves) {
-    const int fb = blk >> 1, r = blk & 1;
+  for (int blk = wave; blk < (NF / 32) * NR; blk += kWaves) {
+    const int fb = blk / NR, r = blk % NR;
     const __bf16* ap = S + (32 * r + lr) * pitch + 32 * fb + kb;
     const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(ap);
     const bf16x8 a1 = *reinterpret_cast<const bf16x8*>(ap + 16);
@@ -471,15 +473,17 @@ __device__ __forceinline__ void zero_acc(f32x16 (&acc)[NR]) {
 // minibatch), then idx_store puts them into rowpN (-1: past the minibatch or a bad index, which
 // is counted in badN and not read).  Split so that the load is waited for well after its issue.
 constexpr long long kNoRow = -(1LL << 62);
+template <int ROWS>
 __device__ __forceinline__ long long idx_load(const F16PPOArgs& a, int t, int tid) {
   long long p = kNoRow;
-  const long r = (long)t * kRows + tid;
-  if (tid < kRows && r < a.mb_rows) p = a.idx[r];
+  const long r = (long)t * ROWS + tid;
+  if (tid < ROWS && r < a.mb_rows) p = a.idx[r];
   return p;
 }
+template <int ROWS>
 __device__ __forceinline__ void idx_store(const F16PPOArgs& a, long long p, long long* rowpN,
                                           float* badN, int tid) {
-  if (tid < kRows) {
+  if (tid < ROWS) {
     float bad = 0.0f;
     if (p == kNoRow) {
       p = -1;
@@ -493,7 +497,7 @@ __device__ __forceinline__ void idx_store(const F16PPOArgs& a, long long p, long
 }
 
 // the rows listed in rowpN as float2 pairs, every load in flight at once
-template <int D, int kPer>
+template <int D, int ROWS, int kPer>
 __device__ __forceinline__ void issue_rows(const F16PPOArgs& a, const long long* rowpN,
                                            float2 (&xr)[kPer], int tid) {
   constexpr int half = D / 2;
@@ -502,7 +506,7 @@ __device__ __forceinline__ void issue_rows(const F16PPOArgs& a, const long long*
     const int it = tid + q * kThreads;
     const int r = it / half, c = it - r * half;
     xr[q] = make_float2(0.0f, 0.0f);
-    if (r < kRows && rowpN[r] >= 0)
+    if (r < ROWS && rowpN[r] >= 0)
       xr[q] = *reinterpret_cast<const float2*>(a.obs + rowpN[r] * a.obs_ld + 2 * c);
   }
 }
@@ -514,39 +518,43 @@ struct HeadIn {
   long long act;
   float old_lp, adv, ret;
 };
+template <int ROWS>
 __device__ __forceinline__ HeadIn gather_head(const F16PPOArgs& a, const long long* rp, int tid) {
   HeadIn h{-1, 0.0f, 0.0f, 0.0f};
   const int lrow = tid >> 3, lch = (tid >> 1) & 3;
-  const long long pr = rp[lrow];
+  const long long pr = lrow < ROWS ? rp[lrow] : -1;
   if (pr >= 0) {
     h.act = a.act[pr * kChan + lch];
     h.old_lp = a.old_logp[pr];
     h.adv = a.adv[pr];
   }
-  if (tid < kRows && rp[tid] >= 0) h.ret = a.ret[rp[tid]];
+  if (tid < ROWS && rp[tid] >= 0) h.ret = a.ret[rp[tid]];
   return h;
 }
 
-// The fused kernel is persistent: one workgroup per CU walks the minibatch's 64-row tiles, and
+// The fused kernel is persistent: one workgroup per CU walks the minibatch's tiles of 64 rows (32
+// in a minibatch too small to give every CU one: fused_tile_rows), and
 // the next tile's gathered rows and loss-head inputs are loaded into registers during the
 // current tile's loss head, landing while it computes.
-template <int KP>
-__global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs a, const Work w) {
+template <int KP, int ROWS>
+__global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs a,
+                                                                const Work w) {
   constexpr int XP = KP + 8;
   constexpr int D = KP == 192 ? 184 : 214;
+  constexpr int NR = ROWS / 32;                           // 32-row MFMA tiles
   constexpr int half = D / 2;                             // float2 per observation row
-  constexpr int kPer = (kRows * half + kThreads - 1) / kThreads;
-  __shared__ __align__(16) __bf16 Xs[kRows * XP];
-  __shared__ __align__(16) __bf16 H1s[kRows * kHPitch];
-  __shared__ __align__(16) __bf16 H2s[kRows * kHPitch];
-  __shared__ __align__(16) float Ls[kRows * kLPitch];     // logits, then (bf16) their gradients
-  __shared__ float rowf[kRows][8];
-  __shared__ float vpart[kWaves][kRows];                  // per-wave partial critic values
-  __shared__ long long rowp[kRows], rowpN[kRows];
+  constexpr int kPer = (ROWS * half + kThreads - 1) / kThreads;
+  __shared__ __align__(16) __bf16 Xs[ROWS * XP];
+  __shared__ __align__(16) __bf16 H1s[ROWS * kHPitch];
+  __shared__ __align__(16) __bf16 H2s[ROWS * kHPitch];
+  __shared__ __align__(16) float Ls[ROWS * kLPitch];     // logits, then (bf16) their gradients
+  __shared__ float rowf[ROWS][8];
+  __shared__ float vpart[kWaves][ROWS];                  // per-wave partial critic values
+  __shared__ long long rowp[ROWS], rowpN[ROWS];
   __shared__ __align__(16) float cst[kB3C];               // biases and the value head, wf[0, kB3C)
-  __shared__ float badN[kRows];
+  __shared__ float badN[ROWS];
   __bf16* Zs = reinterpret_cast<__bf16*>(Ls);
-  static_assert(kRows * kZPitch * 2 <= kRows * kLPitch * 4, "logit gradients overlay the logits");
+  static_assert(ROWS * kZPitch * 2 <= ROWS * kLPitch * 4, "logit gradients overlay the logits");
 
   const long ld = w.ld;
   const __bf16* wbf = static_cast<const __bf16*>(a.wbf);
@@ -563,10 +571,10 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
   float2 xr[kPer];
   int tile = blockIdx.x;
   if (tile >= w.nwg) return;                               // uniform per workgroup
-  idx_store(a, idx_load(a, tile, (int)threadIdx.x), rowpN, badN, (int)threadIdx.x);
+  idx_store<ROWS>(a, idx_load<ROWS>(a, tile, (int)threadIdx.x), rowpN, badN, (int)threadIdx.x);
   __syncthreads();
-  issue_rows<D, kPer>(a, rowpN, xr, (int)threadIdx.x);
-  HeadIn hnext = gather_head(a, rowpN, (int)threadIdx.x);
+  issue_rows<D, ROWS>(a, rowpN, xr, (int)threadIdx.x);
+  HeadIn hnext = gather_head<ROWS>(a, rowpN, (int)threadIdx.x);
   WPre<KP> pa1;
   wprefetch(pa1, wbf + Blob<KP>::W1, 32 * __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6),
             (int)threadIdx.x & 63);
@@ -580,53 +588,53 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lr = lane & 31, lh = (lane >> 5) * 4;
-    const long m0 = (long)tile * kRows;
+    const long m0 = (long)tile * ROWS;
     // ---- stage this tile's rows (normalised at collection), rounded to bf16
-    if (tid < kRows) { rowp[tid] = rowpN[tid]; rowf[tid][7] = badN[tid]; }
+    if (tid < ROWS) { rowp[tid] = rowpN[tid]; rowf[tid][7] = badN[tid]; }
 #pragma unroll
     for (int q = 0; q < kPer; ++q) {
       const int it = tid + q * kThreads;
       const int r = it / half, c = it - r * half;
-      if (r < kRows) {
+      if (r < ROWS) {
         bf16x2 b;
         b[0] = (__bf16)xr[q].x;
         b[1] = (__bf16)xr[q].y;
         *reinterpret_cast<bf16x2*>(Xs + r * XP + 2 * c) = b;
       }
     }
-    for (int it = tid; it < kRows * (KP - D); it += kThreads) {
+    for (int it = tid; it < ROWS * (KP - D); it += kThreads) {
       const int r = it / (KP - D);
       Xs[r * XP + D + (it - r * (KP - D))] = (__bf16)0.0f;
     }
     __syncthreads();
     const int next = tile + gridDim.x;
-    const long long pnext = next < w.nwg ? idx_load(a, next, tid) : kNoRow;
+    const long long pnext = next < w.nwg ? idx_load<ROWS>(a, next, tid) : kNoRow;
     // the loss head's per-row inputs, gathered during the previous tile
     const int item = tid >> 1, hb = tid & 1;           // (row, channel) item, bin half
     const int lrow = item >> 2, lch = item & 3;
     const HeadIn hin = hnext;
-    transpose_t<KP>(Xs, XP, ublock(w.xt, KP, m0), kUBlock, 0, wave, lane);
+    transpose_t<KP, NR>(Xs, XP, ublock(w.xt, KP, m0), kUBlock, 0, wave, lane);
 
     // ---- actor forward
     WPre<kHid> pa2, pl3;
     {
-      f32x16 acc[2];
+      f32x16 acc[NR];
       init_bias_lds(acc, cst + kB1, 32 * wave, lane);
-      gemm_p<2, KP>(acc, pa1, wbf + Blob<KP>::W1, 32 * wave, Xs, XP, lane);
+      gemm_p<NR, KP>(acc, pa1, wbf + Blob<KP>::W1, 32 * wave, Xs, XP, lane);
       wprefetch(pa2, wbf + Blob<KP>::W2A, 32 * wave, lane);
       store_tanh_t(acc, H1s, 32 * wave, ublock(w.h1t, 2 * kHid, m0), kUBlock, 0, lane);
     }
     __syncthreads();
     {
-      f32x16 acc[2];
+      f32x16 acc[NR];
       init_bias_lds(acc, cst + kB2A, 32 * wave, lane);
-      gemm_p<2, kHid>(acc, pa2, wbf + Blob<KP>::W2A, 32 * wave, H1s, kHPitch, lane);
-      if (wave < 6) wprefetch(pl3, wbf + Blob<KP>::W3A, 32 * (wave % 3), lane);
+      gemm_p<NR, kHid>(acc, pa2, wbf + Blob<KP>::W2A, 32 * wave, H1s, kHPitch, lane);
+      if (wave < 3 * NR) wprefetch(pl3, wbf + Blob<KP>::W3A, 32 * (wave % 3), lane);
       store_tanh_t(acc, H2s, 32 * wave, ublock(w.h2t, kHid, m0), kUBlock, 0, lane);
-      idx_store(a, pnext, rowpN, badN, tid);     // the next tile's rows, read after the barrier
+      idx_store<ROWS>(a, pnext, rowpN, badN, tid);     // the next tile's rows, read after the barrier
     }
     __syncthreads();
-    if (wave < 6) {
+    if (wave < 3 * NR) {
       const int ut = wave % 3, rt = wave / 3;
       f32x16 acc[1];
       init_bias_lds(acc, cst + kB3A, 32 * ut, lane);
@@ -654,11 +662,12 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
     const long long act = hin.act;
     const float old_lp = hin.old_lp, adv_r = hin.adv, ret_r = hin.ret;
     if (next < w.nwg) {
-      issue_rows<D, kPer>(a, rowpN, xr, tid);
-      hnext = gather_head(a, rowpN, tid);
+      issue_rows<D, ROWS>(a, rowpN, xr, tid);
+      hnext = gather_head<ROWS>(a, rowpN, tid);
     }
+    const bool head = ROWS == 64 || lrow < ROWS;       // wave-uniform
     float dz[kHalf];
-    {
+    if (head) {
       const long long pr = rowp[lrow];
       const bool valid = pr >= 0;
       const float* l = Ls + lrow * kLPitch + lch * kBins + k0;
@@ -738,31 +747,31 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
     __syncthreads();                          // every logit is read
 #pragma unroll
     for (int k = 0; k < kHalf; ++k)
-      if (k < nb) Zs[lrow * kZPitch + lch * kBins + k0 + k] = (__bf16)dz[k];
-    if (lch == 3 && hb == 1) {
+      if (head && k < nb) Zs[lrow * kZPitch + lch * kBins + k0 + k] = (__bf16)dz[k];
+    if (head && lch == 3 && hb == 1) {
 #pragma unroll
       for (int k = kLogits; k < kLogitsPad; ++k) Zs[lrow * kZPitch + k] = (__bf16)0.0f;
     }
     __syncthreads();
     WPre<kLogitsPad> pb3;
     wprefetch(pb3, wT + kWT3, 32 * wave, lane);
-    transpose_t<kLogitsPad>(Zs, kZPitch, ublock(w.dzt, kLogitsPad, m0), kUBlock, 0, wave, lane);
+    transpose_t<kLogitsPad, NR>(Zs, kZPitch, ublock(w.dzt, kLogitsPad, m0), kUBlock, 0, wave, lane);
 
     // ---- actor backward: dH2 = (dZ W3) (1 - H2^2) in place of H2, dH1 = (dH2 W2) (1 - H1^2)
     WPre<kHid> pb2, pbc, pc2;
     WPre<KP> pc1;
     {
-      f32x16 acc[2];
+      f32x16 acc[NR];
       zero_acc(acc);
-      gemm_p<2, kLogitsPad>(acc, pb3, wT + kWT3, 32 * wave, Zs, kZPitch, lane);
+      gemm_p<NR, kLogitsPad>(acc, pb3, wT + kWT3, 32 * wave, Zs, kZPitch, lane);
       wprefetch(pb2, wT + kWT2A, 32 * wave, lane);
       store_dtanh_t(acc, H2s, H2s, 32 * wave, ublock(w.dh2t, 2 * kHid, m0), kUBlock, 0, lane);
     }
     __syncthreads();
     {
-      f32x16 acc[2];
+      f32x16 acc[NR];
       zero_acc(acc);
-      gemm_p<2, kHid>(acc, pb2, wT + kWT2A, 32 * wave, H2s, kHPitch, lane);
+      gemm_p<NR, kHid>(acc, pb2, wT + kWT2A, 32 * wave, H2s, kHPitch, lane);
       wprefetch(pc1, wbf + Blob<KP>::W1C, 32 * wave, lane);
       store_dtanh_t(acc, H1s, nullptr, 32 * wave, ublock(w.dh1t, 2 * kHid, m0), kUBlock, 0,
                     lane);
@@ -771,20 +780,20 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
 
     // ---- critic forward; the value head is folded into the second layer's epilogue
     {
-      f32x16 acc[2];
+      f32x16 acc[NR];
       init_bias_lds(acc, cst + kB1 + kHid, 32 * wave, lane);
-      gemm_p<2, KP>(acc, pc1, wbf + Blob<KP>::W1C, 32 * wave, Xs, XP, lane);
+      gemm_p<NR, KP>(acc, pc1, wbf + Blob<KP>::W1C, 32 * wave, Xs, XP, lane);
       wprefetch(pc2, wbf + Blob<KP>::W2C, 32 * wave, lane);
       store_tanh_t(acc, H1s, 32 * wave, ublock(w.h1t, 2 * kHid, m0) + kHid * kUBlock, kUBlock, 0,
                    lane);
     }
     __syncthreads();
-    bf16x4 hc2[4][2];                          // this lane's critic layer-2 activations
+    bf16x4 hc2[4][NR];                         // this lane's critic layer-2 activations
     {
-      f32x16 acc[2];
+      f32x16 acc[NR];
       init_bias_lds(acc, cst + kB2C, 32 * wave, lane);
-      gemm_p<2, kHid>(acc, pc2, wbf + Blob<KP>::W2C, 32 * wave, H1s, kHPitch, lane);
-      float vp[2] = {0.0f, 0.0f};
+      gemm_p<NR, kHid>(acc, pc2, wbf + Blob<KP>::W2C, 32 * wave, H1s, kHPitch, lane);
+      float vp[NR] = {};
       float4 w4s[4];
 #pragma unroll
       for (int g = 0; g < 4; ++g)
@@ -793,7 +802,7 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
       for (int g = 0; g < 4; ++g) {
         const float4 w4 = w4s[g];
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
+        for (int r = 0; r < NR; ++r) {
           bf16x4 v;
 #pragma unroll
           for (int j = 0; j < 4; ++j) v[j] = (__bf16)tanh_act(acc[r][4 * g + j]);
@@ -802,11 +811,14 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
         }
       }
 #pragma unroll
-      for (int r = 0; r < 2; ++r) vp[r] += __shfl_xor(vp[r], 32);   // lanes l, l + 32: one row
-      if (lane < 32) { vpart[wave][lr] = vp[0]; vpart[wave][32 + lr] = vp[1]; }
+      for (int r = 0; r < NR; ++r) vp[r] += __shfl_xor(vp[r], 32);   // lanes l, l + 32: one row
+      if (lane < 32) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) vpart[wave][32 * r + lr] = vp[r];
+      }
     }
     __syncthreads();
-    if (tid < kRows) {      // wave 0, one lane per row: value, its error, d(loss)/dv; tile sums
+    if (tid < ROWS) {      // wave 0, one lane per row: value, its error, d(loss)/dv; tile sums
       float v = vpart[0][tid];
 #pragma unroll
       for (int q = 1; q < kWaves; ++q) v += vpart[q][tid];
@@ -821,7 +833,7 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
       // the tile's sums over its rows: pl, ent, kl, cf, se, bad and db3c = sum dv
       float st[7] = {rowf[tid][0], rowf[tid][1], rowf[tid][2], rowf[tid][3], se, rowf[tid][7], dv};
 #pragma unroll
-      for (int q = 0; q < 7; ++q) st[q] = sum64(st[q]);
+      for (int q = 0; q < 7; ++q) st[q] = ROWS == 64 ? sum64(st[q]) : sum32(st[q]);
       if (tid == 0) {
         float* part = w.fpart + (long)tile * kPartCols;
         *reinterpret_cast<float4*>(part) = make_float4(st[0], st[1], st[2], st[3]);
@@ -835,7 +847,9 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
     // units) and dH2c = dv w3c (1 - h2c^2), both from the registers; dH2c to H2s (no reader
     // left since the actor's backward) and unit-major
     {
-      const float dv0 = rowf[lr][4], dv1 = rowf[32 + lr][4];
+      float dv[NR];
+#pragma unroll
+      for (int r = 0; r < NR; ++r) dv[r] = rowf[32 * r + lr][4];
       const UnitMajor out(ublock(w.dh2t, 2 * kHid, m0) + kHid * kUBlock, kUBlock, 0, 32 * wave,
                           lane);
       float* part = w.fpart + (long)tile * kPartCols + kStatCols;
@@ -845,30 +859,33 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
         const float4 w4v = *reinterpret_cast<const float4*>(w3s + unit);
         const float w4[4] = {w4v.x, w4v.y, w4v.z, w4v.w};
         float sw[4];
-        bf16x4 d0, d1;
+        bf16x4 d[NR];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const float h0 = (float)hc2[g][0][j], h1 = (float)hc2[g][1][j];
-          sw[j] = sum32(dv0 * h0 + dv1 * h1);
-          d0[j] = (__bf16)(dv0 * w4[j] * (1.0f - h0 * h0));
-          d1[j] = (__bf16)(dv1 * w4[j] * (1.0f - h1 * h1));
-        }
-        *reinterpret_cast<bf16x4*>(H2s + lr * kHPitch + unit) = d0;
-        *reinterpret_cast<bf16x4*>(H2s + (32 + lr) * kHPitch + unit) = d1;
+          float h[NR];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          out.put(g, 0, j, d0[j]);
-          out.put(g, 1, j, d1[j]);
+          for (int r = 0; r < NR; ++r) {
+            h[r] = (float)hc2[g][r][j];
+            d[r][j] = (__bf16)(dv[r] * w4[j] * (1.0f - h[r] * h[r]));
+          }
+          sw[j] = sum32(NR == 2 ? dv[0] * h[0] + dv[NR - 1] * h[NR - 1] : dv[0] * h[0]);
         }
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          *reinterpret_cast<bf16x4*>(H2s + (32 * r + lr) * kHPitch + unit) = d[r];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int r = 0; r < NR; ++r) out.put(g, r, j, d[r][j]);
         if ((lane & 31) == 0)
           *reinterpret_cast<float4*>(part + unit) = make_float4(sw[0], sw[1], sw[2], sw[3]);
       }
     }
     __syncthreads();
     {
-      f32x16 acc[2];
+      f32x16 acc[NR];
       zero_acc(acc);
-      gemm_p<2, kHid>(acc, pbc, wT + kWT2C, 32 * wave, H2s, kHPitch, lane);
+      gemm_p<NR, kHid>(acc, pbc, wT + kWT2C, 32 * wave, H2s, kHPitch, lane);
       wprefetch(pa1, wbf + Blob<KP>::W1, 32 * wave, lane);    // the next tile's first product
       store_dtanh_t(acc, H1s, nullptr, 32 * wave, ublock(w.dh1t, 2 * kHid, m0) + kHid * kUBlock,
                     kUBlock, 0, lane);
@@ -1451,6 +1468,15 @@ static int wgrad_slots() {
   return slots;
 }
 
+// Rows of a fused-kernel tile.  While 32-row tiles find a CU each, half the work per tile ends
+// sooner (5,000 rows: a minibatch and its optimizer step 86.0 -> 77.0 us); with more of them the
+// weights' stream, the same for a tile of either size, costs more (262,144 rows in 32-row tiles,
+// two workgroups a CU: fused kernel 0.66 ms against 0.50).
+static int fused_tile_rows(long mb_rows) {
+  const long tiles = (mb_rows + 63) / 64 * 2;
+  return tiles <= device_cus() ? 32 : 64;
+}
+
 extern "C" int f16_ppo_param_counts(int obs_dim, long* out2) {
   if (!out2 || (obs_dim != 184 && obs_dim != 214)) return F16_EINVAL;
   const Flat F{obs_dim};
@@ -1475,7 +1501,7 @@ extern "C" int f16_ppo_grad(const F16PPOArgs* a, void* stream) {
   if ((a->obs_ld & 1) || ((uintptr_t)a->obs & 7)) return F16_EINVAL;   // rows move as float2
   const int D = a->obs_dim, kp = (D + 31) / 32 * 32;
   const Flat F{D};
-  const Work w = layout(D, a->mb_rows, a->work, wgrad_slots());
+  const Work w = layout(D, a->mb_rows, a->work, wgrad_slots(), fused_tile_rows(a->mb_rows));
   hipStream_t s = (hipStream_t)stream;
   if (!a->adv_stats) {   // else the epoch's f16_ppo_adv_stats formed them
     hipLaunchKernelGGL(adv_partial_kernel, dim3(w.nadv), dim3(kAdvThreads), 0, s, a->adv, a->idx,
@@ -1484,10 +1510,14 @@ extern "C" int f16_ppo_grad(const F16PPOArgs* a, void* stream) {
                        a->mb_rows, a->count, w.nadv, (const double*)w.advp, w.advs);
   }
   const unsigned fgrid = (unsigned)std::min(w.nwg, device_cus());
-  if (kp == 192)
-    hipLaunchKernelGGL(ppo_fused_kernel<192>, dim3(fgrid), dim3(kThreads), 0, s, *a, w);
+  if (kp == 192 && w.tile_rows == 64)
+    hipLaunchKernelGGL((ppo_fused_kernel<192, 64>), dim3(fgrid), dim3(kThreads), 0, s, *a, w);
+  else if (kp == 192)
+    hipLaunchKernelGGL((ppo_fused_kernel<192, 32>), dim3(fgrid), dim3(kThreads), 0, s, *a, w);
+  else if (w.tile_rows == 64)
+    hipLaunchKernelGGL((ppo_fused_kernel<224, 64>), dim3(fgrid), dim3(kThreads), 0, s, *a, w);
   else
-    hipLaunchKernelGGL(ppo_fused_kernel<224>, dim3(fgrid), dim3(kThreads), 0, s, *a, w);
+    hipLaunchKernelGGL((ppo_fused_kernel<224, 32>), dim3(fgrid), dim3(kThreads), 0, s, *a, w);
   // the four weight-gradient products and their tiles
   WJobs J{};
   const long na = F.na();

@@ -128,6 +128,34 @@ def test_minibatch_grad_matches_oracle(gpu, D, mb, ent_coef, norm_adv):
     assert float(stats[U_.STAT_BAD]) == 0.0
 
 
+@pytest.mark.parametrize("D,mb", [(184, 31), (214, 33), (184, 65), (214, 8191), (184, 8192),
+                                  (184, 8193), (214, 8257), (214, 20001)])
+def test_minibatch_grad_at_tile_edges(gpu, D, mb):
+    """Around the edges of the 32-row tiles (up to 8,192 rows on 256 compute units) and of the
+    64-row tiles above, ragged and whole, with one and several tiles to a workgroup.  The tolerance
+    is the smaller minibatches': the gradients differ from the bf16-mirrored oracle's only by fp32
+    summation order and the bf16 roundings it moves.  The ratios are kept off the clip's edges: a
+    row that such a rounding moves across one enters or leaves the sum of mb random rows, a
+    relative change of about 1 / sqrt(mb) -- 7e-3 at 20,001 rows -- in either implementation."""
+    U = import_pkg("ppo_update")
+    print(f"minibatch grad at tile edges D={D} mb={mb}", flush=True)
+    net = make_net(D, seed=D + mb)
+    flat = flat_of(net)
+    ro, adv, ret = fake_rollout(flat, D, 1, mb + 7, seed=mb, logp_noise=0.0)
+    pick = torch.randint(0, 4, (1, mb + 7), generator=torch.Generator().manual_seed(mb))
+    ro.b_logp += torch.tensor([-0.4, -0.05, 0.05, 0.4])[pick]       # clip range: log 0.8, log 1.2
+    up = U.PPOUpdater(net.to(gpu), U.UpdateConfig(ent_coef=0.01))
+    idx = torch.randperm(mb + 7, generator=torch.Generator().manual_seed(7))[:mb]
+    buf = [x.flatten(0, 1) for x in (ro.b_obs, ro.b_act, ro.b_logp, adv, ret)]
+    up.minibatch_grad(*(x.to(gpu).contiguous() for x in buf), idx.to(gpu))
+    g_ref, st = P.mirror_minibatch(flat, D, *(x[idx] for x in buf), ent_coef=0.01)
+    check_grads(up.grad.cpu(), g_ref, D, tol=3e-3)
+    stats = up.stats[0].cpu()
+    for k, j in (("pl", U.STAT_PL), ("vl", U.STAT_VL), ("ent", U.STAT_ENT), ("kl", U.STAT_KL)):
+        assert math.isclose(float(stats[j]), st[k], rel_tol=2e-3, abs_tol=2e-5), (k, float(stats[j]), st[k])
+    assert float(stats[U.STAT_BAD]) == 0.0
+
+
 def test_out_of_range_indices_are_counted_not_read(gpu):
     U = import_pkg("ppo_update")
     D = 184
