@@ -73,6 +73,10 @@ constexpr int kNormBlockElems = 4096;            // flat elements per squared-no
 constexpr int kWgradSlots = 256;                 // resident wgrad workgroups when the device
                                                  // cannot be asked (1 per CU x 256 CUs)
 constexpr int kMaxChunks = 64;                   // bound on the chunks the partials hold
+constexpr int kHead3 = kLogits * kHid + kLogits;  // the actor head's weights and biases (contiguous
+                                                  // in the flat parameters)
+constexpr int kFusedWG = 256;                    // bound on the fused kernel's workgroups (one per
+                                                 // CU of MI355X), each with a head partial
 
 __host__ __device__ inline long align256(long x) { return (x + 255) & ~255L; }
 
@@ -87,6 +91,7 @@ struct Work {
   double* advp;         // [nadv][2] advantage partial sums
   float* fmid;          // [ceil(nwg / kColRows)][kPartCols] first level of the fpart sums
   float* wpart;         // [nchunk][nflat - 257]
+  float* hpart;         // [fused workgroups][kHead3]: 64-row tiles
   long ld;              // rows, rounded up to 64
   int nwg, nchunk, chunk_rows, nadv, tile_rows;
   long bytes;
@@ -107,7 +112,10 @@ inline long kColGroups(long nrows) { return (nrows + kColRows - 1) / kColRows; }
 
 inline int norm_blocks(long n) { return (int)((n + kNormBlockElems - 1) / kNormBlockElems); }
 
-inline int wgrad_tiles(int kp) { return 2 * ((kp + 255) / 256) + 1 + 1 + 1; }
+// both halves of the first layer, both second layers and, with 32-row tiles, the actor's head
+inline int wgrad_tiles(int kp, int tile_rows) {
+  return 2 * ((kp + 255) / 256) + 1 + 1 + (tile_rows == 32 ? 1 : 0);
+}
 
 inline Work layout(int obs_dim, long mb_rows, void* base, int wg_slots = kWgradSlots,
                    int tile_rows = 64) {
@@ -117,7 +125,7 @@ inline Work layout(int obs_dim, long mb_rows, void* base, int wg_slots = kWgradS
   w.ld = (mb_rows + 63) / 64 * 64;
   w.tile_rows = tile_rows;
   w.nwg = (int)(w.ld / tile_rows);
-  const int tiles = wgrad_tiles(kp);
+  const int tiles = wgrad_tiles(kp, tile_rows);
   // chunks of 64-row stages: one workgroup per resident slot (a grid a little above a
   // multiple of the slots leaves a mostly idle last round), at least 4 stages each
   long chunks = std::max(1, std::min(wg_slots / tiles, kMaxChunks));
@@ -137,15 +145,18 @@ inline Work layout(int obs_dim, long mb_rows, void* base, int wg_slots = kWgradS
   w.normp = reinterpret_cast<double*>(take((long)norm_blocks(F.n()) * 2 * sizeof(double)));
   w.xt = reinterpret_cast<__bf16*>(take((long)kp * w.ld * 2));
   w.h1t = reinterpret_cast<__bf16*>(take(512L * w.ld * 2));
-  w.h2t = reinterpret_cast<__bf16*>(take(256L * w.ld * 2));   // actor layer 2 only
+  // the head's operands (actor layer 2 and the logit gradients) leave only from 32-row tiles
+  const long ld3 = std::min(w.ld, 32L * kFusedWG);
+  w.h2t = reinterpret_cast<__bf16*>(take(256L * ld3 * 2));
   w.dh1t = reinterpret_cast<__bf16*>(take(512L * w.ld * 2));
   w.dh2t = reinterpret_cast<__bf16*>(take(512L * w.ld * 2));
-  w.dzt = reinterpret_cast<__bf16*>(take((long)kLogitsPad * w.ld * 2));
+  w.dzt = reinterpret_cast<__bf16*>(take((long)kLogitsPad * ld3 * 2));
   w.fpart = reinterpret_cast<float*>(take(w.ld / 32 * kPartCols * 4));
   w.nadv = (int)((w.ld + kAdvThreads * kAdvPer - 1) / (kAdvThreads * kAdvPer));
   w.advp = reinterpret_cast<double*>(take((long)w.nadv * 2 * sizeof(double)));
   w.fmid = reinterpret_cast<float*>(take(kColGroups(w.ld / 32) * kPartCols * 4));
   w.wpart = reinterpret_cast<float*>(take(cap * (F.n() - 257) * 4));
+  w.hpart = reinterpret_cast<float*>(take(std::min(w.ld / 64, (long)kFusedWG) * kHead3 * 4));
   w.bytes = off;
   return w;
 }
@@ -393,6 +404,23 @@ __device__ __forceinline__ void store_dtanh_t(const f32x16 (&acc)[NR], const __b
   }
 }
 
+// An MFMA operand of 32 columns x 16 rows of an LDS tile [row][pitch], the rows the summed index:
+// lane l gets column col0 + l % 32 of rows row0 + 8 (l / 32) + 0..7.  Each transposing read gives
+// a 16-lane group 4 rows x 16 columns (lane i names row i / 4, columns 4 (i % 4) + 0..3 and
+// receives column i of the four rows).
+__device__ __forceinline__ bf16x8 tr_frag(const __bf16* S, int pitch, int row0, int col0,
+                                          int lane) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  const int i = lane & 15;
+  const __bf16* p = S + (row0 + 8 * (lane >> 5) + (i >> 2)) * pitch + col0 +
+                    16 * ((lane >> 4) & 1) + 4 * (i & 3);
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 4 * pitch));
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
+  return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
 // A product's first weight fragments, loaded before the previous phase's epilogue.  vmcnt
 // retires loads and stores in issue order, so a weight load issued after that epilogue's global
 // stores could only be waited for behind all of them; these are issued ahead of the stores.
@@ -542,6 +570,12 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
   constexpr int XP = KP + 8;
   constexpr int D = KP == 192 ? 184 : 214;
   constexpr int NR = ROWS / 32;                           // 32-row MFMA tiles
+  // With several tiles to a workgroup the actor head's weight gradient is summed in registers over
+  // them (48 accumulators a lane: this wave's 32 units by the 96 padded logits), so that the second
+  // layer's activations and the logit gradients, 704 bytes a row, need not leave at all:
+  // 262,144 rows 784 -> 732 us for the gradient and the optimizer step.
+  constexpr bool kHeadGrad = ROWS == 64;
+  constexpr int kZT = kLogitsPad / 32;
   constexpr int half = D / 2;                             // float2 per observation row
   constexpr int kPer = (ROWS * half + kThreads - 1) / kThreads;
   __shared__ __align__(16) __bf16 Xs[ROWS * XP];
@@ -568,6 +602,9 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
     reinterpret_cast<float4*>(cst)[i] = reinterpret_cast<const float4*>(wf)[i];
   const float* w3s = cst + kW3C;
 
+  f32x16 hacc[kZT];
+  float hbias = 0.0f;            // waves 0..2: this lane's half sum of logit 32 wave + lane % 32
+  if constexpr (kHeadGrad) zero_acc(hacc);
   float2 xr[kPer];
   int tile = blockIdx.x;
   if (tile >= w.nwg) return;                               // uniform per workgroup
@@ -630,7 +667,10 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
       init_bias_lds(acc, cst + kB2A, 32 * wave, lane);
       gemm_p<NR, kHid>(acc, pa2, wbf + Blob<KP>::W2A, 32 * wave, H1s, kHPitch, lane);
       if (wave < 3 * NR) wprefetch(pl3, wbf + Blob<KP>::W3A, 32 * (wave % 3), lane);
-      store_tanh_t(acc, H2s, 32 * wave, ublock(w.h2t, kHid, m0), kUBlock, 0, lane);
+      if constexpr (kHeadGrad)
+        store_tanh(acc, H2s, 32 * wave, lane);
+      else
+        store_tanh_t(acc, H2s, 32 * wave, ublock(w.h2t, kHid, m0), kUBlock, 0, lane);
       idx_store<ROWS>(a, pnext, rowpN, badN, tid);     // the next tile's rows, read after the barrier
     }
     __syncthreads();
@@ -755,7 +795,26 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
     __syncthreads();
     WPre<kLogitsPad> pb3;
     wprefetch(pb3, wT + kWT3, 32 * wave, lane);
-    transpose_t<kLogitsPad, NR>(Zs, kZPitch, ublock(w.dzt, kLogitsPad, m0), kUBlock, 0, wave, lane);
+    if constexpr (kHeadGrad) {
+      // dW3 += dZ^T H2 over the tile's rows: this wave's own units of H2, which it alone replaces
+      // below
+#pragma unroll
+      for (int k = 0; k < ROWS / 16; ++k) {
+        const bf16x8 hb2 = tr_frag(H2s, kHPitch, 16 * k, 32 * wave, lane);
+#pragma unroll
+        for (int t = 0; t < kZT; ++t) {
+          const bf16x8 z = tr_frag(Zs, kZPitch, 16 * k, 32 * t, lane);
+          hacc[t] = mfma(z, hb2, hacc[t]);
+          if (wave == t) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) hbias += (float)z[i];
+          }
+        }
+      }
+    } else {
+      transpose_t<kLogitsPad, NR>(Zs, kZPitch, ublock(w.dzt, kLogitsPad, m0), kUBlock, 0, wave,
+                                  lane);
+    }
 
     // ---- actor backward: dH2 = (dZ W3) (1 - H2^2) in place of H2, dH1 = (dH2 W2) (1 - H1^2)
     WPre<kHid> pb2, pbc, pc2;
@@ -892,6 +951,20 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
     }
     // the next tile first writes Xs, rowp and rowf (read before the syncs above) and H1s only
     // after its first barrier, so no barrier is needed here
+  }
+  if constexpr (kHeadGrad) {
+    float* hp = w.hpart + (long)blockIdx.x * kHead3;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+    for (int t = 0; t < kZT; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int z = 32 * t + 8 * (e >> 2) + (lane >> 5) * 4 + (e & 3);
+        if (z < kLogits) hp[z * kHid + 32 * wave + (lane & 31)] = hacc[t][e];
+      }
+    hbias += __shfl_xor(hbias, 32);
+    const int z = 32 * wave + lane;
+    if (wave < kZT && lane < 32 && z < kLogits) hp[kLogits * kHid + z] = hbias;
   }
 }
 
@@ -1063,16 +1136,58 @@ __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long
   }
 }
 
+// The actor head's partials (64-row tiles): the last blocks of a column-sum launch add them over
+// the fused kernel's workgroups, VW columns to a thread, 16 row phases combined in order, and the
+// other blocks leave the head's columns alone (kHead3 and its offset are multiples of 4).
+struct HeadSum {
+  const float* part;    // [nrows][kHead3]
+  int nrows;            // 0: the head is among the other columns
+  int blk0;             // first block of the head
+  long c0;              // its flat offset
+  __device__ __forceinline__ bool holds(long c) const {
+    return nrows > 0 && c >= c0 && c < c0 + kHead3;
+  }
+};
+template <int VW>
+__device__ __forceinline__ void head_colsum(const float* __restrict__ part, int nrows, int blk,
+                                            float* __restrict__ out) {
+  typedef float vec __attribute__((ext_vector_type(VW)));
+  constexpr int kCols = 16, kPh = 256 / kCols;       // threads across the columns, row phases
+  __shared__ vec s[kPh][kCols];
+  const int t = threadIdx.x % kCols, ph = threadIdx.x / kCols;
+  const int c = VW * (blk * kCols + t);
+  vec acc = {};
+  if (c < kHead3) {
+#pragma unroll 4
+    for (int r = ph; r < nrows; r += kPh)
+      acc += *reinterpret_cast<const vec*>(part + (long)r * kHead3 + c);
+  }
+  s[ph][t] = acc;
+  __syncthreads();
+  if (ph == 0 && c < kHead3) {
+    vec v = s[0][t];
+#pragma unroll
+    for (int k = 1; k < kPh; ++k) v += s[k][t];
+    *reinterpret_cast<vec*>(out + c) = v;
+  }
+}
+
 // out[c] = sum over r of part[r * ld + c], rows in a fixed order: PH row phases per column
 template <int PH>
 __global__ __launch_bounds__(64 * PH) void colsum_kernel(const float* __restrict__ part, int nrows,
                                                          long ld, long ncols,
-                                                         float* __restrict__ out) {
+                                                         float* __restrict__ out,
+                                                         const HeadSum head) {
+  static_assert(PH == 4, "the head's blocks are of 256 threads");
+  if (head.nrows > 0 && (int)blockIdx.x >= head.blk0) {
+    head_colsum<1>(head.part, head.nrows, blockIdx.x - head.blk0, out + head.c0);
+    return;
+  }
   __shared__ float s[PH][64];
   const int t = threadIdx.x & 63, ph = threadIdx.x >> 6;
   const long c = (long)blockIdx.x * 64 + t;
   float acc = 0.0f;
-  if (c < ncols)
+  if (c < ncols && !head.holds(c))
     for (int r = ph; r < nrows; r += PH) acc += part[(long)r * ld + c];
   s[ph][t] = acc;
   __syncthreads();
@@ -1080,7 +1195,7 @@ __global__ __launch_bounds__(64 * PH) void colsum_kernel(const float* __restrict
     float v = s[0][t];
 #pragma unroll
     for (int k = 1; k < PH; ++k) v += s[k][t];
-    out[c] = v;
+    if (!head.holds(c)) out[c] = v;
   }
 }
 
@@ -1088,12 +1203,17 @@ __global__ __launch_bounds__(64 * PH) void colsum_kernel(const float* __restrict
 // 4, part and out 16-byte aligned): every column summed in the same row order, the same bits
 __global__ __launch_bounds__(256) void colsum4_kernel(const float* __restrict__ part, int nrows,
                                                       long ld, long ncols,
-                                                      float* __restrict__ out) {
+                                                      float* __restrict__ out,
+                                                      const HeadSum head) {
+  if (head.nrows > 0 && (int)blockIdx.x >= head.blk0) {
+    head_colsum<4>(head.part, head.nrows, blockIdx.x - head.blk0, out + head.c0);
+    return;
+  }
   __shared__ float4 s[4][64];
   const int t = threadIdx.x & 63, ph = threadIdx.x >> 6;
   const long c = 4 * ((long)blockIdx.x * 64 + t);
   float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (c < ncols)
+  if (c < ncols && !head.holds(c))
     for (int r = ph; r < nrows; r += 4) {
       const float4 v = *reinterpret_cast<const float4*>(part + (long)r * ld + c);
       acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
@@ -1107,7 +1227,7 @@ __global__ __launch_bounds__(256) void colsum4_kernel(const float* __restrict__ 
       const float4 u = s[k][t];
       v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
     }
-    *reinterpret_cast<float4*>(out + c) = v;
+    if (!head.holds(c)) *reinterpret_cast<float4*>(out + c) = v;
   }
 }
 
@@ -1474,7 +1594,7 @@ static int wgrad_slots() {
 // two workgroups a CU: fused kernel 0.66 ms against 0.50).
 static int fused_tile_rows(long mb_rows) {
   const long tiles = (mb_rows + 63) / 64 * 2;
-  return tiles <= device_cus() ? 32 : 64;
+  return tiles <= std::min(device_cus(), kFusedWG) ? 32 : 64;
 }
 
 extern "C" int f16_ppo_param_counts(int obs_dim, long* out2) {
@@ -1509,7 +1629,7 @@ extern "C" int f16_ppo_grad(const F16PPOArgs* a, void* stream) {
     hipLaunchKernelGGL(adv_final_kernel, dim3(1), dim3(kAdvThreads), 0, s, a->adv, a->idx,
                        a->mb_rows, a->count, w.nadv, (const double*)w.advp, w.advs);
   }
-  const unsigned fgrid = (unsigned)std::min(w.nwg, device_cus());
+  const unsigned fgrid = (unsigned)std::min(w.nwg, std::min(device_cus(), kFusedWG));
   if (kp == 192 && w.tile_rows == 64)
     hipLaunchKernelGGL((ppo_fused_kernel<192, 64>), dim3(fgrid), dim3(kThreads), 0, s, *a, w);
   else if (kp == 192)
@@ -1534,7 +1654,8 @@ extern "C" int f16_ppo_grad(const F16PPOArgs* a, void* stream) {
   (void)na;
   int nt = 0;
   const int ntA[4] = {2, 1, 1, 1}, ntB[4] = {(kp + 255) / 256, 1, 1, 1};
-  for (int j = 0; j < 4; ++j)
+  const int njob = w.tile_rows == 32 ? 4 : 3;   // else the fused kernel summed the head's
+  for (int j = 0; j < njob; ++j)
     for (int ta = 0; ta < ntA[j]; ++ta)
       for (int tb = 0; tb < ntB[j]; ++tb) {
         J.tj[nt] = (unsigned char)j;
@@ -1570,12 +1691,16 @@ extern "C" int f16_ppo_grad(const F16PPOArgs* a, void* stream) {
   const long pld = F.n() - 257;          // every flat parameter but the critic's value head
   hipLaunchKernelGGL(wgrad_kernel, dim3(nt * w.nchunk), dim3(kWThreads), 0, s, J, w.ld,
                      w.chunk_rows, w.wpart, pld);
-  if (pld % 4 == 0 && ((uintptr_t)a->grad & 15) == 0)
-    hipLaunchKernelGGL(colsum4_kernel, dim3((unsigned)((pld / 4 + 63) / 64)), dim3(256), 0, s,
-                       (const float*)w.wpart, w.nchunk, pld, pld, a->grad);
+  const int vw = pld % 4 == 0 && ((uintptr_t)a->grad & 15) == 0 ? 4 : 1;
+  const int cblk = (int)((pld / vw + 63) / 64);
+  HeadSum head{w.hpart, w.tile_rows == 64 ? (int)fgrid : 0, cblk, F.a_w3()};
+  const int hblk = head.nrows > 0 ? (kHead3 / vw + 15) / 16 : 0;
+  if (vw == 4)
+    hipLaunchKernelGGL(colsum4_kernel, dim3((unsigned)(cblk + hblk)), dim3(256), 0, s,
+                       (const float*)w.wpart, w.nchunk, pld, pld, a->grad, head);
   else
-    hipLaunchKernelGGL(colsum_kernel<4>, dim3((unsigned)((pld + 63) / 64)), dim3(256), 0, s,
-                       (const float*)w.wpart, w.nchunk, pld, pld, a->grad);
+    hipLaunchKernelGGL(colsum_kernel<4>, dim3((unsigned)(cblk + hblk)), dim3(256), 0, s,
+                       (const float*)w.wpart, w.nchunk, pld, pld, a->grad, head);
   // the per-workgroup partials (statistics, dw3c, db3c): groups of kColRows rows, then the groups
   const int ng = (int)kColGroups(w.nwg);
   hipLaunchKernelGGL(colsum_group_kernel, dim3((kPartCols + 63) / 64, ng), dim3(256), 0, s,
