@@ -1,24 +1,27 @@
 // ppo_kernels.hip -- the PPO update of the discrete actor-critic MLP on gfx950.
 //
-// One minibatch (f16_ppo_grad) is seven launches:
-//   adv_partial/final  minibatch advantage mean and sample std (shifted fp64 sums, two levels);
-//   ppo_fused_kernel   per 64 gathered rows (persistent, one workgroup per CU, the next tile's
-//                      rows in flight during the current one): forward of both networks, the loss head (softmax,
-//                      log-probability, entropy, ratio, clipped surrogate, value error) and the
-//                      backward chain down to the first hidden layer, all with the rows'
-//                      activations held in LDS.  The layer inputs and output gradients every
-//                      weight gradient needs leave unit-major ([feature][row], bf16), so the
-//                      reduction over rows reads them as contiguous MFMA fragments;
-//   wgrad_kernel       every weight gradient dW = dY^T X as one split-K launch: 256 x 256 output
-//                      tiles of all four products, rows in chunks, 64-row stages double-buffered
-//                      through LDS, fp32 partials per chunk (bias gradients are the row sums of
-//                      dY, taken while staging);
-//   colsum kernels     the partials summed in a fixed order (deterministic, no atomics): the
-//                      weight-gradient chunks, then the fused kernel's per-tile rows in two
-//                      levels, the second (colsum_tail_kernel) also forming the minibatch means.
-// The optimizer step (f16_ppo_adam_step) is three: per-block squared-norm partials, the clipped
-// Adam update (every block re-reduces the norm partials in the same order), and the repack of
-// the bf16 blobs the rollout and the next minibatch read.
+// One minibatch (f16_ppo_grad) is four launches, three where the caller has the advantages'
+// statistics (seven in the arrangement before: 262,144 rows 732 -> 717 us with the optimizer step):
+//   adv_partial        the partial sums of the minibatch advantage mean and sample std (shifted
+//                      fp64 sums; the fused kernel merges them);
+//   ppo_fused_kernel   per 64 gathered rows (32 in a small minibatch; persistent, one workgroup per
+//                      CU, the next tile's rows in flight during the current one): forward of both
+//                      networks, the loss head (softmax, log-probability, entropy, ratio, clipped
+//                      surrogate, value error) and the backward chain down to the first hidden
+//                      layer, all with the rows' activations held in LDS.  The layer inputs and
+//                      output gradients the hidden layers' weight gradients need leave unit-major
+//                      ([feature][row], bf16), so the reduction over rows reads them as contiguous
+//                      MFMA fragments; the heads' weight gradients and the statistics are summed
+//                      over a workgroup's tiles on the chip, one partial per workgroup;
+//   wgrad_kernel       the hidden layers' weight gradients dW = dY^T X as one split-K launch:
+//                      256 x 256 output tiles of all products, rows in chunks, 64-row stages
+//                      double-buffered through LDS, fp32 partials per chunk (bias gradients are the
+//                      row sums of dY, taken while staging);
+//   colsum4_kernel     every partial summed in a fixed order (deterministic, no atomics), and the
+//                      minibatch means formed from the statistics.
+// The optimizer step (f16_ppo_adam_step) is two: per-block squared-norm partials, and the clipped
+// Adam update (every block re-reduces the norm partials in the same order), which also writes the
+// bf16 blobs the rollout and the next minibatch read.
 //
 // The forward runs the same tiles, the same K order and the same epilogue as the rollout kernel
 // (policy_mfma.h), and the log-probability is formed with the same expression sequence, so at
@@ -87,9 +90,8 @@ struct Work {
                                                 // kp, 512, 256, 512, 512, kLogitsPad
                                                 // (h2t: the actor's layer 2; the critic's
                                                 // enters only the value head, summed in-kernel)
-  float* fpart;         // [nwg][kPartCols]
+  float* fpart;         // [fused workgroups][kPartCols]
   double* advp;         // [nadv][2] advantage partial sums
-  float* fmid;          // [ceil(nwg / kColRows)][kPartCols] first level of the fpart sums
   float* wpart;         // [nchunk][nflat - 257]
   float* hpart;         // [fused workgroups][kHead3]: 64-row tiles
   long ld;              // rows, rounded up to 64
@@ -106,9 +108,6 @@ constexpr long kUBlock = 64;
 __host__ __device__ inline __bf16* ublock(__bf16* buf, long nf, long m0) {
   return buf + (m0 / kUBlock) * nf * kUBlock + m0 % kUBlock;
 }
-
-constexpr int kColRows = 64;                     // rows per block of the two-level column sum
-inline long kColGroups(long nrows) { return (nrows + kColRows - 1) / kColRows; }
 
 inline int norm_blocks(long n) { return (int)((n + kNormBlockElems - 1) / kNormBlockElems); }
 
@@ -151,10 +150,9 @@ inline Work layout(int obs_dim, long mb_rows, void* base, int wg_slots = kWgradS
   w.dh1t = reinterpret_cast<__bf16*>(take(512L * w.ld * 2));
   w.dh2t = reinterpret_cast<__bf16*>(take(512L * w.ld * 2));
   w.dzt = reinterpret_cast<__bf16*>(take((long)kLogitsPad * ld3 * 2));
-  w.fpart = reinterpret_cast<float*>(take(w.ld / 32 * kPartCols * 4));
+  w.fpart = reinterpret_cast<float*>(take(std::min(w.ld / 32, (long)kFusedWG) * kPartCols * 4));
   w.nadv = (int)((w.ld + kAdvThreads * kAdvPer - 1) / (kAdvThreads * kAdvPer));
   w.advp = reinterpret_cast<double*>(take((long)w.nadv * 2 * sizeof(double)));
-  w.fmid = reinterpret_cast<float*>(take(kColGroups(w.ld / 32) * kPartCols * 4));
   w.wpart = reinterpret_cast<float*>(take(cap * (F.n() - 257) * 4));
   w.hpart = reinterpret_cast<float*>(take(std::min(w.ld / 64, (long)kFusedWG) * kHead3 * 4));
   w.bytes = off;
@@ -164,7 +162,7 @@ inline Work layout(int obs_dim, long mb_rows, void* base, int wg_slots = kWgradS
 // ---- minibatch advantage mean and sample standard deviation (ppo_gpu.py:2077-2078): each block
 // sums (x - K) and (x - K)^2 in fp64 over its rows, K the minibatch's first advantage (shifting
 // keeps the one-pass variance exact to fp64 rounding for any mean); one block merges the partials
-// in a fixed order.
+// in a fixed order (adv_merge).
 __device__ __forceinline__ void adv_partial_body(const float* __restrict__ adv,
                                                  const long long* __restrict__ idx, int n,
                                                  long count, double* __restrict__ part, int blk) {
@@ -210,38 +208,31 @@ __global__ __launch_bounds__(kAdvThreads) void adv_partial_kernel(const float* _
   adv_partial_body(adv, idx, n, count, part, blockIdx.x);
 }
 
-__device__ __forceinline__ void adv_final_body(const float* __restrict__ adv,
-                                               const long long* __restrict__ idx, int n,
-                                               long count, int nblk,
-                                               const double* __restrict__ part, float* advs) {
-  __shared__ double rs[kAdvThreads], rq[kAdvThreads];
+// The merge of a minibatch's partials by the first wavefront of a workgroup: mean and std to
+// out2[0], out2[1] in LDS, visible to every thread on return.
+__device__ __forceinline__ void adv_merge(const float* __restrict__ adv,
+                                          const long long* __restrict__ idx, int n, long count,
+                                          int nblk, const double* __restrict__ part, float* out2) {
   const int t = threadIdx.x;
-  double s = 0.0, q = 0.0;
-  for (int b = t; b < nblk; b += kAdvThreads) { s += part[2L * b]; q += part[2L * b + 1]; }
-  rs[t] = s;
-  rq[t] = q;
-  __syncthreads();
-  for (int w = kAdvThreads / 2; w > 0; w >>= 1) {
-    if (t < w) { rs[t] += rs[t + w]; rq[t] += rq[t + w]; }
-    __syncthreads();
-  }
-  if (t == 0) {
+  if (t < 64) {
     const long long p0 = idx[0];
     const double K = (p0 >= 0 && p0 < count) ? (double)adv[p0] : 0.0;
-    const double ms = rs[0] / n;                       // mean of the shifted values
-    double var = n > 1 ? (rq[0] - rs[0] * ms) / (n - 1) : 0.0;
-    var = var < 0.0 ? 0.0 : var;
-    advs[0] = (float)(K + ms);
-    advs[1] = (float)sqrt(var);
+    double s = 0.0, q = 0.0;
+    for (int b = t; b < nblk; b += 64) { s += part[2L * b]; q += part[2L * b + 1]; }
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) {
+      s += __shfl_xor(s, w);
+      q += __shfl_xor(q, w);
+    }
+    if (t == 0) {
+      const double ms = s / n;                           // mean of the shifted values
+      double var = n > 1 ? (q - s * ms) / (n - 1) : 0.0;
+      var = var < 0.0 ? 0.0 : var;
+      out2[0] = (float)(K + ms);
+      out2[1] = (float)sqrt(var);
+    }
   }
-}
-
-__global__ __launch_bounds__(kAdvThreads) void adv_final_kernel(const float* __restrict__ adv,
-                                                                const long long* __restrict__ idx,
-                                                                int n, long count, int nblk,
-                                                                const double* __restrict__ part,
-                                                                float* advs) {
-  adv_final_body(adv, idx, n, count, nblk, part, advs);
+  __syncthreads();
 }
 
 // The same for every minibatch of an epoch at once: minibatch j (blockIdx.y, then blockIdx.x of
@@ -258,9 +249,11 @@ __global__ __launch_bounds__(kAdvThreads) void adv_partial_epoch_kernel(
 __global__ __launch_bounds__(kAdvThreads) void adv_final_epoch_kernel(
     const float* __restrict__ adv, const long long* __restrict__ idx, int mb, long total,
     long count, int nadv, const double* __restrict__ part, float* __restrict__ out) {
+  __shared__ float ms[2];
   const long s0 = (long)blockIdx.x * mb;
-  adv_final_body(adv, idx + s0, (int)min((long)mb, total - s0), count, nadv,
-                 part + 2L * nadv * blockIdx.x, out + 2L * blockIdx.x);
+  adv_merge(adv, idx + s0, (int)min((long)mb, total - s0), count, nadv,
+            part + 2L * nadv * blockIdx.x, ms);
+  if (threadIdx.x < 2) out[2L * blockIdx.x + threadIdx.x] = ms[threadIdx.x];
 }
 
 // ---- fused forward / loss / backward of 64 gathered rows
@@ -587,6 +580,7 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
   __shared__ long long rowp[ROWS], rowpN[ROWS];
   __shared__ __align__(16) float cst[kB3C];               // biases and the value head, wf[0, kB3C)
   __shared__ float badN[ROWS];
+  __shared__ float psum[kPartCols];                       // this workgroup's partial row
   __bf16* Zs = reinterpret_cast<__bf16*>(Ls);
   static_assert(ROWS * kZPitch * 2 <= ROWS * kLPitch * 4, "logit gradients overlay the logits");
 
@@ -595,11 +589,10 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
   const __bf16* wT = static_cast<const __bf16*>(a.wT);
   const float* wf = a.wf;
   const float inv_mb = 1.0f / (float)a.mb_rows;
-  // launch constants read once (scalar loads before any store of this kernel)
-  const float* const am = a.adv_stats ? a.adv_stats : w.advs;
-  const float adv_mean = am[0], adv_std = am[1], b3c = wf[kB3C];
+  const float b3c = wf[kB3C];
   for (int i = threadIdx.x; i < kB3C / 4; i += kThreads)
     reinterpret_cast<float4*>(cst)[i] = reinterpret_cast<const float4*>(wf)[i];
+  for (int i = threadIdx.x; i < kPartCols; i += kThreads) psum[i] = 0.0f;
   const float* w3s = cst + kW3C;
 
   f32x16 hacc[kZT];
@@ -615,6 +608,21 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
   WPre<KP> pa1;
   wprefetch(pa1, wbf + Blob<KP>::W1, 32 * __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6),
             (int)threadIdx.x & 63);
+  // the minibatch's advantage statistics: given, or merged here by every workgroup from the partials
+  // (a launch less; the first writes them down for the minibatch's means) while the rows load
+  float adv_mean, adv_std;
+  if (a.adv_stats) {
+    adv_mean = a.adv_stats[0];
+    adv_std = a.adv_stats[1];
+  } else {
+    adv_merge(a.adv, a.idx, a.mb_rows, a.count, w.nadv, w.advp, &vpart[0][0]);
+    auto uniform = [](float x) {
+      return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
+    };
+    adv_mean = uniform(vpart[0][0]);
+    adv_std = uniform(vpart[0][1]);
+    if (blockIdx.x == 0 && threadIdx.x < 2) w.advs[threadIdx.x] = vpart[0][threadIdx.x];
+  }
   // every load above has landed before the loop, so the loop's own waits for the gathered rows
   // count only the previous tile's loads (they retire by its last product's final wait)
   __builtin_amdgcn_s_waitcnt(0x0F70);                     // vmcnt(0)
@@ -894,10 +902,11 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
 #pragma unroll
       for (int q = 0; q < 7; ++q) st[q] = ROWS == 64 ? sum64(st[q]) : sum32(st[q]);
       if (tid == 0) {
-        float* part = w.fpart + (long)tile * kPartCols;
-        *reinterpret_cast<float4*>(part) = make_float4(st[0], st[1], st[2], st[3]);
-        *reinterpret_cast<float4*>(part + 4) = make_float4(0.0f, st[4], 0.0f, st[5]);
-        part[kStatCols + kHid] = st[6];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) psum[q] += st[q];
+        psum[5] += st[4];
+        psum[7] += st[5];
+        psum[kStatCols + kHid] += st[6];
       }
     }
     __syncthreads();
@@ -911,7 +920,7 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
       for (int r = 0; r < NR; ++r) dv[r] = rowf[32 * r + lr][4];
       const UnitMajor out(ublock(w.dh2t, 2 * kHid, m0) + kHid * kUBlock, kUBlock, 0, 32 * wave,
                           lane);
-      float* part = w.fpart + (long)tile * kPartCols + kStatCols;
+      float* part = psum + kStatCols;
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int unit = 32 * wave + 8 * g + lh;
@@ -936,8 +945,10 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
         for (int j = 0; j < 4; ++j)
 #pragma unroll
           for (int r = 0; r < NR; ++r) out.put(g, r, j, d[r][j]);
-        if ((lane & 31) == 0)
-          *reinterpret_cast<float4*>(part + unit) = make_float4(sw[0], sw[1], sw[2], sw[3]);
+        if ((lane & 31) == 0) {             // the only lane that adds to these units
+#pragma unroll
+          for (int j = 0; j < 4; ++j) part[unit + j] += sw[j];
+        }
       }
     }
     __syncthreads();
@@ -952,6 +963,9 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
     // the next tile first writes Xs, rowp and rowf (read before the syncs above) and H1s only
     // after its first barrier, so no barrier is needed here
   }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kPartCols; i += kThreads)
+    w.fpart[(long)blockIdx.x * kPartCols + i] = psum[i];
   if constexpr (kHeadGrad) {
     float* hp = w.hpart + (long)blockIdx.x * kHead3;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1136,6 +1150,52 @@ __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long
   }
 }
 
+// The fused kernel's partial rows: statistics, dw3c and db3c, one row per workgroup.  The last
+// blocks of a column-sum launch add them, 16 columns to a block and 16 row phases combined in
+// order; the first also forms the minibatch means from its statistics sums
+// (ppo_gpu.py:2080-2081, 2098, 2107-2108).
+struct TailSum {
+  const float* part;    // [nrows][kPartCols]
+  int nrows;
+  int blk0;             // first of the kTailBlocks blocks
+  const float* advs;    // mean and std of the advantages
+  int n;                // minibatch rows
+  float* grad_w3c;
+  float* stats;
+};
+constexpr int kTailBlocks = (kStatCols + kHid + 1 + 15) / 16;
+__device__ __forceinline__ void tail_colsum(const TailSum& T, int blk) {
+  __shared__ float s[16][17];
+  const int t = threadIdx.x % 16, ph = threadIdx.x / 16;
+  const int c = blk * 16 + t;                          // below kPartCols
+  static_assert(kTailBlocks * 16 <= kPartCols, "the blocks' columns are in the row");
+  float acc = 0.0f;
+#pragma unroll 4
+  for (int r = ph; r < T.nrows; r += 16) acc += T.part[(long)r * kPartCols + c];
+  s[ph][t] = acc;
+  __syncthreads();
+  if (ph == 0) {
+    float v = s[0][t];
+#pragma unroll
+    for (int k = 1; k < 16; ++k) v += s[k][t];
+    s[0][t] = v;
+    if (c >= kStatCols && c < kStatCols + kHid + 1) T.grad_w3c[c - kStatCols] = v;
+  }
+  if (blk != 0) return;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const float fn = (float)T.n;
+    T.stats[F16_PPO_STAT_POLICY_LOSS] = s[0][0] / fn;
+    T.stats[F16_PPO_STAT_ENTROPY] = s[0][1] / fn;
+    T.stats[F16_PPO_STAT_APPROX_KL] = s[0][2] / fn;
+    T.stats[F16_PPO_STAT_CLIPFRAC] = s[0][3] / fn;
+    T.stats[F16_PPO_STAT_VALUE_LOSS] = 0.5f * (s[0][5] / fn);
+    T.stats[F16_PPO_STAT_ADV_MEAN] = T.advs[0];
+    T.stats[F16_PPO_STAT_ADV_STD] = T.advs[1];
+    T.stats[7] = s[0][7];
+  }
+}
+
 // The actor head's partials (64-row tiles): the last blocks of a column-sum launch add them over
 // the fused kernel's workgroups, VW columns to a thread, 16 row phases combined in order, and the
 // other blocks leave the head's columns alone (kHead3 and its offset are multiples of 4).
@@ -1177,7 +1237,11 @@ template <int PH>
 __global__ __launch_bounds__(64 * PH) void colsum_kernel(const float* __restrict__ part, int nrows,
                                                          long ld, long ncols,
                                                          float* __restrict__ out,
-                                                         const HeadSum head) {
+                                                         const HeadSum head, const TailSum tail) {
+  if ((int)blockIdx.x >= tail.blk0) {
+    tail_colsum(tail, blockIdx.x - tail.blk0);
+    return;
+  }
   static_assert(PH == 4, "the head's blocks are of 256 threads");
   if (head.nrows > 0 && (int)blockIdx.x >= head.blk0) {
     head_colsum<1>(head.part, head.nrows, blockIdx.x - head.blk0, out + head.c0);
@@ -1204,7 +1268,11 @@ __global__ __launch_bounds__(64 * PH) void colsum_kernel(const float* __restrict
 __global__ __launch_bounds__(256) void colsum4_kernel(const float* __restrict__ part, int nrows,
                                                       long ld, long ncols,
                                                       float* __restrict__ out,
-                                                      const HeadSum head) {
+                                                      const HeadSum head, const TailSum tail) {
+  if ((int)blockIdx.x >= tail.blk0) {
+    tail_colsum(tail, blockIdx.x - tail.blk0);
+    return;
+  }
   if (head.nrows > 0 && (int)blockIdx.x >= head.blk0) {
     head_colsum<4>(head.part, head.nrows, blockIdx.x - head.blk0, out + head.c0);
     return;
@@ -1231,77 +1299,23 @@ __global__ __launch_bounds__(256) void colsum4_kernel(const float* __restrict__ 
   }
 }
 
-// first level over the fused kernel's partial rows: block (x, y) sums rows [64y, 64y + 64) of
-// columns [64x, 64x + 64) (4 phases of 16 rows, combined in order)
-__global__ __launch_bounds__(256) void colsum_group_kernel(const float* __restrict__ part, int nrows,
-                                                           float* __restrict__ mid) {
-  __shared__ float sm[4][64];
-  const int t = threadIdx.x & 63, ph = threadIdx.x >> 6;
-  const int c = blockIdx.x * 64 + t;
-  const int r0 = blockIdx.y * kColRows;
-  float acc = 0.0f;
-  if (c < kPartCols)
-    for (int r = r0 + ph; r < min(r0 + kColRows, nrows); r += 4) acc += part[(long)r * kPartCols + c];
-  sm[ph][t] = acc;
-  __syncthreads();
-  if (ph == 0 && c < kPartCols)
-    mid[(long)blockIdx.y * kPartCols + c] = (sm[0][t] + sm[1][t]) + (sm[2][t] + sm[3][t]);
-}
-
-// second level over the first-level sums `mid` ([ng][kPartCols]): block x sums columns
-// [64x, 64x + 64) exactly as colsum_kernel<4> does (row phases r = ph (mod 4), combined in
-// order); the statistics columns [0, kStatCols) go to sums, dw3c and db3c to grad; block 0 then
-// forms the minibatch means from its statistics sums (ppo_gpu.py:2080-2081, 2098, 2107-2108).
-__global__ __launch_bounds__(256) void colsum_tail_kernel(const float* __restrict__ mid, int ng,
-                                                          float* __restrict__ sums,
-                                                          float* __restrict__ grad_w3c,
-                                                          const float* __restrict__ advs, int n,
-                                                          float* __restrict__ stats) {
-  __shared__ float sm[4][64];
-  const int t = threadIdx.x & 63, ph = threadIdx.x >> 6;
-  const int c = blockIdx.x * 64 + t;
-  constexpr int kCols = kStatCols + kHid + 1;
-  float acc = 0.0f;
-  if (c < kCols)
-    for (int r = ph; r < ng; r += 4) acc += mid[(long)r * kPartCols + c];
-  sm[ph][t] = acc;
-  __syncthreads();
-  if (ph == 0 && c < kCols) {
-    float v = sm[0][t];
-#pragma unroll
-    for (int k = 1; k < 4; ++k) v += sm[k][t];
-    if (c < kStatCols) {
-      sums[c] = v;
-      sm[0][t] = v;
-    } else {
-      grad_w3c[c - kStatCols] = v;
-    }
-  }
-  if (blockIdx.x != 0) return;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const float fn = (float)n;
-    stats[F16_PPO_STAT_POLICY_LOSS] = sm[0][0] / fn;
-    stats[F16_PPO_STAT_ENTROPY] = sm[0][1] / fn;
-    stats[F16_PPO_STAT_APPROX_KL] = sm[0][2] / fn;
-    stats[F16_PPO_STAT_CLIPFRAC] = sm[0][3] / fn;
-    stats[F16_PPO_STAT_VALUE_LOSS] = 0.5f * (sm[0][5] / fn);
-    stats[F16_PPO_STAT_ADV_MEAN] = advs[0];
-    stats[F16_PPO_STAT_ADV_STD] = advs[1];
-    stats[7] = sm[0][7];
-  }
-}
-
 // ---- clip_grad_norm_ + Adam
 __global__ __launch_bounds__(256) void sumsq_kernel(const float* __restrict__ g, long n, long na,
                                                     double* __restrict__ normp) {
   __shared__ double sa[256], sc[256];
   const long b0 = (long)blockIdx.x * kNormBlockElems;
   double xa = 0.0, xc = 0.0;
-  for (int i = threadIdx.x; i < kNormBlockElems; i += 256) {
-    const long k = b0 + i;
+  // every load in flight at once (elements past the end read the last and are not summed): loaded
+  // one at a time behind the range check they took 8 us at 0.25 M parameters
+  constexpr int kPer = kNormBlockElems / 256;
+  float x[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) x[i] = g[min(b0 + threadIdx.x + 256L * i, n - 1)];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const long k = b0 + threadIdx.x + 256L * i;
+    const double v = x[i];
     if (k < n) {
-      const double v = g[k];
       if (k < na) xa += v * v;
       else xc += v * v;
     }
@@ -1322,11 +1336,73 @@ struct AdamScalars {
   float one_m_b1, b2, one_m_b2, eps, max_norm;
 };
 
+// element (n, k) of a matrix [N][K] in the fragment-major blobs (policy_mfma.h)
+template <long K>
+__device__ __forceinline__ long frag(long n, long k) {
+  return ((n >> 5) * (K >> 4) + (k >> 4)) * 512 + ((((k >> 3) & 1) << 5) + (n & 31)) * 8 + (k & 7);
+}
+// The blobs' copies of flat parameter k (the inverse of pack_kernel's gather).
+template <int KP>
+__device__ __forceinline__ void scatter_param(long k, float x, __bf16* __restrict__ wbf,
+                                              float* __restrict__ wf, __bf16* __restrict__ wT) {
+  constexpr long D = KP == 192 ? 184 : 214;
+  const Flat F{D};
+  const bool critic = k >= F.na();
+  const long q = critic ? k - F.na() : k;          // the two networks' first layers are alike
+  const __bf16 b = (__bf16)x;
+  if (q < 256 * D) {
+    if (wbf) wbf[Blob<KP>::W1 + frag<KP>((critic ? kHid : 0) + q / D, q % D)] = b;
+    return;
+  }
+  const long u = q - 256 * D;                      // b1 [256], W2 [256][256], b2 [256], W3, b3
+  if (u < 256) {
+    if (wf) wf[kB1 + (critic ? kHid : 0) + u] = x;
+  } else if (u < 256 + 65536) {
+    const long n = (u - 256) >> 8, c = (u - 256) & 255;
+    if (wbf) wbf[(critic ? Blob<KP>::W2C : Blob<KP>::W2A) + frag<kHid>(n, c)] = b;
+    if (wT) wT[(critic ? kWT2C : kWT2A) + frag<kHid>(c, n)] = b;
+  } else if (u < 66048) {
+    if (wf) wf[(critic ? kB2C : kB2A) + u - 65792] = x;
+  } else if (critic) {
+    if (wf) wf[u < 66304 ? kW3C + u - 66048 : kB3C] = x;
+  } else if (u < 87552) {
+    const long n = (u - 66048) >> 8, c = (u - 66048) & 255;
+    if (wbf) wbf[Blob<KP>::W3A + frag<kHid>(n, c)] = b;
+    if (wT) wT[kWT3 + frag<kLogitsPad>(c, n)] = b;
+  } else {
+    if (wf) wf[kB3A + u - 87552] = x;
+  }
+}
+// the blobs' padding, element j of kPads: zero as pack_kernel leaves it
+template <int KP>
+struct Pads {
+  static constexpr long D = KP == 192 ? 184 : 214;
+  static constexpr long kX = 512 * (KP - D), kZ = (long)(kLogitsPad - kLogits) * kHid;
+  static constexpr long kPads = kX + kZ + kLogitsPad - kLogits;
+  static __device__ __forceinline__ void zero(long j, __bf16* wbf, float* wf, __bf16* wT) {
+    if (j < kX) {
+      if (wbf) wbf[Blob<KP>::W1 + frag<KP>(j / (KP - D), D + j % (KP - D))] = (__bf16)0.0f;
+    } else if (j < kX + kZ) {
+      const long n = kLogits + (j - kX) / kHid, c = (j - kX) % kHid;
+      if (wbf) wbf[Blob<KP>::W3A + frag<kHid>(n, c)] = (__bf16)0.0f;
+      if (wT) wT[kWT3 + frag<kLogitsPad>(c, n)] = (__bf16)0.0f;
+    } else if (j < kPads) {
+      if (wf) wf[kB3A + kLogits + j - kX - kZ] = 0.0f;
+    }
+  }
+};
+
+// Each updated parameter leaves for the blobs too, where a launch of its own read them all back
+// (one of the four launches fewer that took a 5,000-row gradient and step from 77.0 to 63.6 us).
+template <int KP>
 __global__ __launch_bounds__(256) void adam_kernel(float* __restrict__ p, float* __restrict__ m,
                                                    float* __restrict__ v, float* __restrict__ g,
                                                    long n, long na, const double* __restrict__ normp,
                                                    int nblk, const AdamScalars S,
-                                                   float* __restrict__ norms_out) {
+                                                   float* __restrict__ norms_out,
+                                                   __bf16* __restrict__ wbf,
+                                                   float* __restrict__ wf,
+                                                   __bf16* __restrict__ wT) {
   __shared__ double sa[256], sc[256];
   __shared__ float clip[2];
   double xa = 0.0, xc = 0.0;
@@ -1348,7 +1424,10 @@ __global__ __launch_bounds__(256) void adam_kernel(float* __restrict__ p, float*
   }
   __syncthreads();
   const long k = (long)blockIdx.x * 256 + threadIdx.x;
-  if (k >= n) return;
+  if (k >= n) {
+    Pads<KP>::zero(k - n, wbf, wf, wT);
+    return;
+  }
   const int net = k < na ? 0 : 1;
   const float gk = g[k] * clip[net];
   g[k] = gk;
@@ -1357,7 +1436,9 @@ __global__ __launch_bounds__(256) void adam_kernel(float* __restrict__ p, float*
   vk = vk * S.b2;                              // exp_avg_sq.mul_(beta2)
   vk = vk + S.one_m_b2 * gk * gk;              //   .addcmul_(grad, grad, 1 - beta2)
   const float denom = sqrtf(vk) / S.bc2_sqrt + S.eps;
-  p[k] = p[k] + S.lr_step[net] * (mk / denom); // param.addcdiv_(exp_avg, denom, -step_size)
+  const float pk = p[k] + S.lr_step[net] * (mk / denom);   // param.addcdiv_(exp_avg, denom, -step_size)
+  p[k] = pk;
+  scatter_param<KP>(k, pk, wbf, wf, wT);
   m[k] = mk;
   v[k] = vk;
 }
@@ -1623,12 +1704,9 @@ extern "C" int f16_ppo_grad(const F16PPOArgs* a, void* stream) {
   const Flat F{D};
   const Work w = layout(D, a->mb_rows, a->work, wgrad_slots(), fused_tile_rows(a->mb_rows));
   hipStream_t s = (hipStream_t)stream;
-  if (!a->adv_stats) {   // else the epoch's f16_ppo_adv_stats formed them
+  if (!a->adv_stats)     // else the epoch's f16_ppo_adv_stats formed them
     hipLaunchKernelGGL(adv_partial_kernel, dim3(w.nadv), dim3(kAdvThreads), 0, s, a->adv, a->idx,
                        a->mb_rows, a->count, w.advp);
-    hipLaunchKernelGGL(adv_final_kernel, dim3(1), dim3(kAdvThreads), 0, s, a->adv, a->idx,
-                       a->mb_rows, a->count, w.nadv, (const double*)w.advp, w.advs);
-  }
   const unsigned fgrid = (unsigned)std::min(w.nwg, std::min(device_cus(), kFusedWG));
   if (kp == 192 && w.tile_rows == 64)
     hipLaunchKernelGGL((ppo_fused_kernel<192, 64>), dim3(fgrid), dim3(kThreads), 0, s, *a, w);
@@ -1695,19 +1773,16 @@ extern "C" int f16_ppo_grad(const F16PPOArgs* a, void* stream) {
   const int cblk = (int)((pld / vw + 63) / 64);
   HeadSum head{w.hpart, w.tile_rows == 64 ? (int)fgrid : 0, cblk, F.a_w3()};
   const int hblk = head.nrows > 0 ? (kHead3 / vw + 15) / 16 : 0;
+  const TailSum tail{w.fpart, (int)fgrid, cblk + hblk,
+                     a->adv_stats ? a->adv_stats : (const float*)w.advs, a->mb_rows,
+                     a->grad + F.c_w3(), a->stats};
+  const dim3 cgrid((unsigned)(cblk + hblk + kTailBlocks));
   if (vw == 4)
-    hipLaunchKernelGGL(colsum4_kernel, dim3((unsigned)(cblk + hblk)), dim3(256), 0, s,
-                       (const float*)w.wpart, w.nchunk, pld, pld, a->grad, head);
+    hipLaunchKernelGGL(colsum4_kernel, cgrid, dim3(256), 0, s,
+                       (const float*)w.wpart, w.nchunk, pld, pld, a->grad, head, tail);
   else
-    hipLaunchKernelGGL(colsum_kernel<4>, dim3((unsigned)(cblk + hblk)), dim3(256), 0, s,
-                       (const float*)w.wpart, w.nchunk, pld, pld, a->grad, head);
-  // the per-workgroup partials (statistics, dw3c, db3c): groups of kColRows rows, then the groups
-  const int ng = (int)kColGroups(w.nwg);
-  hipLaunchKernelGGL(colsum_group_kernel, dim3((kPartCols + 63) / 64, ng), dim3(256), 0, s,
-                     (const float*)w.fpart, w.nwg, w.fmid);
-  hipLaunchKernelGGL(colsum_tail_kernel, dim3((kStatCols + kHid + 1 + 63) / 64), dim3(256), 0, s,
-                     (const float*)w.fmid, ng, w.advs + 8, a->grad + F.c_w3(),
-                     a->adv_stats ? a->adv_stats : (const float*)w.advs, a->mb_rows, a->stats);
+    hipLaunchKernelGGL(colsum_kernel<4>, cgrid, dim3(256), 0, s,
+                       (const float*)w.wpart, w.nchunk, pld, pld, a->grad, head, tail);
   return f16_last_error();
 }
 
@@ -1734,13 +1809,17 @@ extern "C" int f16_ppo_adam_step(const F16AdamArgs* a, void* stream) {
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(sumsq_kernel, dim3(nblk), dim3(256), 0, s, (const float*)a->grad, n, F.na(),
                      w.normp);
-  hipLaunchKernelGGL(adam_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a->param,
-                     a->exp_avg, a->exp_avg_sq, a->grad, n, F.na(), (const double*)w.normp, nblk, S,
-                     a->grad_norms);
-  int rc = f16_last_error();
-  if (rc || (!a->wbf && !a->wT)) return rc;
-  return a->obs_dim == 184 ? launch_pack<192>(a->param, a->wbf, a->wf, a->wT, s)
-                           : launch_pack<224>(a->param, a->wbf, a->wf, a->wT, s);
+  auto adam = [&](auto kern, long pads) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)((n + pads + 255) / 256)), dim3(256), 0, s, a->param,
+                       a->exp_avg, a->exp_avg_sq, a->grad, n, F.na(), (const double*)w.normp, nblk,
+                       S, a->grad_norms, static_cast<__bf16*>(a->wbf), a->wf,
+                       static_cast<__bf16*>(a->wT));
+  };
+  if (a->obs_dim == 184)
+    adam(adam_kernel<192>, Pads<192>::kPads);
+  else
+    adam(adam_kernel<224>, Pads<224>::kPads);
+  return f16_last_error();
 }
 
 extern "C" int f16_ppo_pack(const float* param, int obs_dim, void* wbf, float* wf, void* wT,

@@ -196,6 +196,22 @@ def test_optimizer_step_matches_torch_adam(gpu):
     assert torch.equal(net.packed()[0], wbf) and torch.equal(net.packed()[1], wf)
 
 
+@pytest.mark.parametrize("D", [184, 214])
+def test_optimizer_step_writes_whole_blobs(gpu, D):
+    """The step leaves the blobs as f16_ppo_pack makes them from the stepped parameters, every
+    element and the padding (the blobs hold NaN before)."""
+    U = import_pkg("ppo_update")
+    up = U.PPOUpdater(make_net(D, seed=5).to(gpu))
+    up.grad.copy_(torch.randn(up.grad.numel(), generator=torch.Generator().manual_seed(D)))
+    for b in (up.wbf, up.wf, up.wT):
+        b.fill_(float("nan"))
+    up.optimizer_step()
+    got = [b.clone() for b in (up.wbf, up.wf, up.wT)]
+    up.pack()
+    for name, g, b in zip(("wbf", "wf", "wT"), got, (up.wbf, up.wf, up.wT)):
+        assert torch.equal(g, b), name
+
+
 def test_update_matches_reference_loop(gpu):
     """Two epochs of four minibatches (ragged last) with fixed permutations: final parameters,
     statistics and norms against the reference loop with the mirrored gradients."""
