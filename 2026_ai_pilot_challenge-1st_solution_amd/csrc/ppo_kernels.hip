@@ -1005,11 +1005,12 @@ struct WJob {
   int wld;             // flat row length of W
 };
 
-constexpr int kWMaxWG = 8 * kMaxChunks;   // tiles x chunks (at most 8 tiles)
+constexpr int kWMaxTiles = 9;             // 128-feature tiles of all four products
+constexpr int kWMaxWG = kWMaxTiles * kMaxChunks;
 
 struct WJobs {
   WJob job[4];
-  unsigned char tj[8], ta[8], tb[8];
+  unsigned char tj[kWMaxTiles], ta[kWMaxTiles], tb[kWMaxTiles];
   int ntiles;
   // workgroup i computes tile wg[i] >> 6 of chunk wg[i] & 63.  Workgroups go to the 8 XCDs round
   // robin (i to XCD i % 8): the two tiles that read the same layer-input rows (the two 256-unit
@@ -1019,14 +1020,17 @@ struct WJobs {
 
 static_assert(kWK == kUBlock, "a weight-gradient stage is one 64-row block of each operand");
 
+template <int TA>
 __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long mp,
                                                              int chunk_rows, float* __restrict__ wpart,
                                                              long pld) {
-  __shared__ __align__(16) __bf16 As[2][kWT * kWPitch];
+  constexpr int kPA = kWPieces * TA / kWT;    // A's 16-byte pieces per thread
+  constexpr int NI = TA / 64;                 // 32-feature blocks of A per wave
+  __shared__ __align__(16) __bf16 As[2][TA * kWPitch];
   __shared__ __align__(16) __bf16 Bs[2][kWT * kWPitch];
   const int tile = J.wg[blockIdx.x] >> 6, c = J.wg[blockIdx.x] & 63;
   const WJob& jb = J.job[J.tj[tile]];
-  const int fa0 = kWT * J.ta[tile], fb0 = kWT * J.tb[tile];
+  const int fa0 = TA * J.ta[tile], fb0 = kWT * J.tb[tile];
   const bool bias = J.tb[tile] == 0;
   const long k0 = (long)c * chunk_rows;
   const long k1 = min(k0 + chunk_rows, mp);
@@ -1035,10 +1039,10 @@ __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wa = wave & 1, wb = wave >> 1;
   const int part = tid & 7;                   // 8-row piece of a feature's 64 rows
-  bf16x8 ra[kWPieces], rb[kWPieces];
-  float bsum[kWPieces];
+  bf16x8 ra[kPA], rb[kWPieces];
+  float bsum[kPA];
 #pragma unroll
-  for (int q = 0; q < kWPieces; ++q) bsum[q] = 0.0f;
+  for (int q = 0; q < kPA; ++q) bsum[q] = 0.0f;
   // one block of an operand is one buffer window of its present features: the pieces past them
   // read as zero by the window's bound, so every load of a stage is issued without a branch
   const int off0 = 2 * ((tid >> 3) * (int)kUBlock + 8 * part);
@@ -1055,7 +1059,8 @@ __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long
 #pragma unroll
     for (int q = 0; q < kWPieces; ++q) {
       const int off = off0 + q * (kWThreads / 8) * (int)kUBlock * 2;
-      ra[q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(ba, off, 0, 0));
+      if (q < kPA)
+        ra[q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(ba, off, 0, 0));
       rb[q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(bb, off, 0, 0));
     }
     __builtin_amdgcn_sched_barrier(0);          // issued here, not sunk to the stage's end
@@ -1064,12 +1069,12 @@ __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long
 #pragma unroll
     for (int q = 0; q < kWPieces; ++q) {
       const int f = (tid >> 3) + (kWThreads / 8) * q;
-      *reinterpret_cast<bf16x8*>(&As[buf][f * kWPitch + 8 * part]) = ra[q];
+      if (q < kPA) *reinterpret_cast<bf16x8*>(&As[buf][f * kWPitch + 8 * part]) = ra[q];
       *reinterpret_cast<bf16x8*>(&Bs[buf][f * kWPitch + 8 * part]) = rb[q];
     }
     if (bias) {
 #pragma unroll
-      for (int q = 0; q < kWPieces; ++q)
+      for (int q = 0; q < kPA; ++q)
 #pragma unroll
         for (int i = 0; i < 8; ++i) bsum[q] += (float)ra[q][i];
     }
@@ -1078,10 +1083,10 @@ __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long
   // MFMA runs, those of absent features on zeros: a branch around each one kept the LDS reads of
   // a slice behind the slice before it (262,144 rows: 275 -> 269 us; 5,000 rows: 22.8 -> 21.9).
   // What is left is the operands' stream, 20 bytes per ns and CU at either size.
-  const bool live = fa0 + 128 * wa < jb.nA && fb0 + 64 * wb < jb.nB;
-  f32x16 acc[4][2];
+  const bool live = fa0 + (TA / 2) * wa < jb.nA && fb0 + 64 * wb < jb.nB;
+  f32x16 acc[NI][2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -1096,12 +1101,12 @@ __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long
     const int buf = st & 1;
     if (st + 1 < nst) load(st + 1);
     if (live) {
-      const __bf16* ap = &As[buf][(128 * wa + lr) * kWPitch + lk];
+      const __bf16* ap = &As[buf][((TA / 2) * wa + lr) * kWPitch + lk];
       const __bf16* bp = &Bs[buf][(64 * wb + lr) * kWPitch + lk];
-      bf16x8 af[2][4], bfg[2][2];               // one K slice ahead of the MFMAs
+      bf16x8 af[2][NI], bfg[2][2];               // one K slice ahead of the MFMAs
       auto frags = [&](int kk) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < NI; ++i)
           af[kk & 1][i] = *reinterpret_cast<const bf16x8*>(ap + 32 * i * kWPitch + 16 * kk);
 #pragma unroll
         for (int j = 0; j < 2; ++j)
@@ -1113,7 +1118,7 @@ __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long
         if (kk + 1 < kWK / 16) frags(kk + 1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < NI; ++i)
 #pragma unroll
           for (int j = 0; j < 2; ++j)
             acc[i][j] = mfma(af[kk & 1][i], bfg[kk & 1][j], acc[i][j]);
@@ -1123,23 +1128,23 @@ __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long
     __syncthreads();
   }
   float* out = wpart + (long)c * pld;
-  // element e of acc[i][j]: a = fa0 + 128wa + 32i + 8(e/4) + 4(lane/32) + e%4, b = fb0 + 64wb + 32j + lane%32
+  // element e of acc[i][j]: a = fa0 + (TA / 2) wa + 32i + 8(e/4) + 4(lane/32) + e%4, b = fb0 + 64wb + 32j + lane%32
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int b = fb0 + 64 * wb + 32 * j + lr;
       if (b >= jb.vB) continue;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int aa = fa0 + 128 * wa + 32 * i + 8 * (e >> 2) + (lane >> 5) * 4 + (e & 3);
+        const int aa = fa0 + (TA / 2) * wa + 32 * i + 8 * (e >> 2) + (lane >> 5) * 4 + (e & 3);
         if (aa < jb.vA)
           out[jb.wbase[aa >> 8] + (long)(aa & 255) * jb.wld + b] = acc[i][j][e];
       }
     }
   if (bias) {
 #pragma unroll
-    for (int q = 0; q < kWPieces; ++q) {
+    for (int q = 0; q < kPA; ++q) {
       float s = bsum[q];
       s += __shfl_xor(s, 1);
       s += __shfl_xor(s, 2);
@@ -1661,7 +1666,7 @@ static int wgrad_slots() {
   static int slots = 0;
   if (slots == 0) {
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgrad_kernel, kWThreads, 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgrad_kernel<kWT>, kWThreads, 0) !=
             hipSuccess || per_cu < 1)
       per_cu = 1;
     slots = per_cu * device_cus();
@@ -1730,9 +1735,18 @@ extern "C" int f16_ppo_grad(const F16PPOArgs* a, void* stream) {
                   {F.a_w3(), F.a_w3()},
                   {F.a_b3(), F.a_b3()}, 256};
   (void)na;
-  int nt = 0;
-  const int ntA[4] = {2, 1, 1, 1}, ntB[4] = {(kp + 255) / 256, 1, 1, 1};
   const int njob = w.tile_rows == 32 ? 4 : 3;   // else the fused kernel summed the head's
+  int nt = 0;
+  // Halves of the 256-feature A side while they too find a CU each: a stage is bound by the bytes
+  // a CU streams, and half a tile has 48 KB of 64 and half the results to write (5,000 rows: 22.0 -> 16.0 us).
+  // In a larger minibatch B's second reading costs more than the idle CUs.
+  const int ntile128 = 8 + (njob == 4 ? 1 : 0);
+  const int TA = ntile128 * w.nchunk <= wgrad_slots() ? 128 : kWT;
+  int ntA[4], ntB[4];
+  for (int j = 0; j < 4; ++j) {
+    ntA[j] = (J.job[j].nA + TA - 1) / TA;
+    ntB[j] = (J.job[j].nB + kWT - 1) / kWT;
+  }
   for (int j = 0; j < njob; ++j)
     for (int ta = 0; ta < ntA[j]; ++ta)
       for (int tb = 0; tb < ntB[j]; ++tb) {
@@ -1745,10 +1759,10 @@ extern "C" int f16_ppo_grad(const F16PPOArgs* a, void* stream) {
   {
     // tiles 0 and 1 (job 0's A halves, one B) of chunk c at ids 16 (c / 8) + c % 8 and 8 more,
     // the other tiles' work in the ids left, in tile-major order; where the last pair would not
-    // fit the grid (few chunks), id c nt + t runs tile t of chunk c
+    // fit the grid (few chunks) or the tiles are halves, id c nt + t runs tile t of chunk c
     const int nwg = nt * w.nchunk;
     const int last = 16 * ((w.nchunk - 1) / 8) + (w.nchunk - 1) % 8 + 8;
-    if (last < nwg) {
+    if (TA == kWT && last < nwg) {
       for (int i = 0; i < nwg; ++i) J.wg[i] = 0xffff;
       for (int c = 0; c < w.nchunk; ++c) {
         const int id0 = 16 * (c / 8) + c % 8;
@@ -1767,8 +1781,12 @@ extern "C" int f16_ppo_grad(const F16PPOArgs* a, void* stream) {
     }
   }
   const long pld = F.n() - 257;          // every flat parameter but the critic's value head
-  hipLaunchKernelGGL(wgrad_kernel, dim3(nt * w.nchunk), dim3(kWThreads), 0, s, J, w.ld,
-                     w.chunk_rows, w.wpart, pld);
+  if (TA == kWT)
+    hipLaunchKernelGGL(wgrad_kernel<kWT>, dim3(nt * w.nchunk), dim3(kWThreads), 0, s, J, w.ld,
+                       w.chunk_rows, w.wpart, pld);
+  else
+    hipLaunchKernelGGL(wgrad_kernel<128>, dim3(nt * w.nchunk), dim3(kWThreads), 0, s, J, w.ld,
+                       w.chunk_rows, w.wpart, pld);
   const int vw = pld % 4 == 0 && ((uintptr_t)a->grad & 15) == 0 ? 4 : 1;
   const int cblk = (int)((pld / vw + 63) / 64);
   HeadSum head{w.hpart, w.tile_rows == 64 ? (int)fgrid : 0, cblk, F.a_w3()};
