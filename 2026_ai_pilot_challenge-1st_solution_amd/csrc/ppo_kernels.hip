@@ -95,7 +95,7 @@ struct Work {
   float* wpart;         // [nchunk][nflat - 257]
   float* hpart;         // [fused workgroups][kHead3]: 64-row tiles
   long ld;              // rows, rounded up to 64
-  int nwg, nchunk, chunk_rows, nadv, tile_rows;
+  int nwg, nchunk, nadv, tile_rows;
   long bytes;
 };
 
@@ -131,7 +131,6 @@ inline Work layout(int obs_dim, long mb_rows, void* base, int wg_slots = kWgradS
   long cr = (w.ld + chunks - 1) / chunks;
   cr = (cr + 63) / 64 * 64;
   if (cr < 256) cr = 256;
-  w.chunk_rows = (int)cr;
   w.nchunk = (int)((w.ld + cr - 1) / cr);
   // partial rows are allocated for min(ceil(ld / 256), kMaxChunks) chunks: never fewer than
   // nchunk (cr >= 256, nchunk <= chunks) and non-decreasing in ld, so a workspace sized for a
@@ -1022,7 +1021,7 @@ static_assert(kWK == kUBlock, "a weight-gradient stage is one 64-row block of ea
 
 template <int TA>
 __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long mp,
-                                                             int chunk_rows, float* __restrict__ wpart,
+                                                             int nchunk, float* __restrict__ wpart,
                                                              long pld) {
   constexpr int kPA = kWPieces * TA / kWT;    // A's 16-byte pieces per thread
   constexpr int NI = TA / 64;                 // 32-feature blocks of A per wave
@@ -1032,9 +1031,11 @@ __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long
   const WJob& jb = J.job[J.tj[tile]];
   const int fa0 = TA * J.ta[tile], fb0 = kWT * J.tb[tile];
   const bool bias = J.tb[tile] == 0;
-  const long k0 = (long)c * chunk_rows;
-  const long k1 = min(k0 + chunk_rows, mp);
-  const int nst = k1 > k0 ? (int)((k1 - k0) / kWK) : 0;
+  // Chunk c takes the 64-row blocks c, c + nchunk, ... counted from the minibatch's end: the rows the
+  // fused kernel wrote last are read first, while the infinity cache still holds them (262,144
+  // rows: 229 -> 202 us).
+  const int nblk = (int)(mp / kUBlock);
+  const int nst = nblk > c ? (nblk - c + nchunk - 1) / nchunk : 0;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wa = wave & 1, wb = wave >> 1;
@@ -1048,9 +1049,15 @@ __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long
   const int off0 = 2 * ((tid >> 3) * (int)kUBlock + 8 * part);
   const int bytesA = max(0, jb.nA - fa0) * (int)kUBlock * 2;
   const int bytesB = max(0, jb.nB - fb0) * (int)kUBlock * 2;
-  const __bf16* const A0 = jb.A + (k0 / kUBlock) * jb.sA + fa0 * kUBlock;
-  const __bf16* const B0 = jb.B + (k0 / kUBlock) * jb.sB + fb0 * kUBlock;
-  const long sA = jb.sA, sB = jb.sB;
+  const __bf16* const A0 = jb.A + (long)(nblk - 1 - c) * jb.sA + fa0 * kUBlock;
+  const __bf16* const B0 = jb.B + (long)(nblk - 1 - c) * jb.sB + fb0 * kUBlock;
+  const long sA = -jb.sA * nchunk, sB = -jb.sB * nchunk;
+  // Operands read once are read past the caches (non-temporal), which leaves the rows still to come
+  // in them (with the order above 202 -> 176 us); a layer input that two tiles of an XCD share stays
+  // cached (read past the caches too, 65,536 rows 53 -> 58 us), and so does all that half tiles read
+  // (5,000 rows: 16.0 against 17.3 us).
+  constexpr int kNT = TA == kWT ? 2 : 0;
+  const bool shared = jb.nA > kWT;
   auto load = [&](int st) {                     // kWK = 64: one block per stage
     const __amdgpu_buffer_rsrc_t ba = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<__bf16*>(A0 + st * sA), 0, bytesA, kBufWord3);
@@ -1060,8 +1067,21 @@ __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long
     for (int q = 0; q < kWPieces; ++q) {
       const int off = off0 + q * (kWThreads / 8) * (int)kUBlock * 2;
       if (q < kPA)
-        ra[q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(ba, off, 0, 0));
-      rb[q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(bb, off, 0, 0));
+        ra[q] = __builtin_bit_cast(bf16x8,
+                                   __builtin_amdgcn_raw_buffer_load_b128(ba, off, 0, kNT));
+    }
+    if (kNT == 0 || shared) {
+#pragma unroll
+      for (int q = 0; q < kWPieces; ++q)
+        rb[q] = __builtin_bit_cast(
+            bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                        bb, off0 + q * (kWThreads / 8) * (int)kUBlock * 2, 0, 0));
+    } else {
+#pragma unroll
+      for (int q = 0; q < kWPieces; ++q)
+        rb[q] = __builtin_bit_cast(
+            bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                        bb, off0 + q * (kWThreads / 8) * (int)kUBlock * 2, 0, kNT));
     }
     __builtin_amdgcn_sched_barrier(0);          // issued here, not sunk to the stage's end
   };
@@ -1082,7 +1102,7 @@ __global__ __launch_bounds__(kWThreads, 1) void wgrad_kernel(const WJobs J, long
   // A wave none of whose block is present features multiplies nothing.  Inside a live wave every
   // MFMA runs, those of absent features on zeros: a branch around each one kept the LDS reads of
   // a slice behind the slice before it (262,144 rows: 275 -> 269 us; 5,000 rows: 22.8 -> 21.9).
-  // What is left is the operands' stream, 20 bytes per ns and CU at either size.
+  // What is left is the operands' stream.
   const bool live = fa0 + (TA / 2) * wa < jb.nA && fb0 + 64 * wb < jb.nB;
   f32x16 acc[NI][2];
 #pragma unroll
@@ -1783,10 +1803,10 @@ extern "C" int f16_ppo_grad(const F16PPOArgs* a, void* stream) {
   const long pld = F.n() - 257;          // every flat parameter but the critic's value head
   if (TA == kWT)
     hipLaunchKernelGGL(wgrad_kernel<kWT>, dim3(nt * w.nchunk), dim3(kWThreads), 0, s, J, w.ld,
-                       w.chunk_rows, w.wpart, pld);
+                       w.nchunk, w.wpart, pld);
   else
     hipLaunchKernelGGL(wgrad_kernel<128>, dim3(nt * w.nchunk), dim3(kWThreads), 0, s, J, w.ld,
-                       w.chunk_rows, w.wpart, pld);
+                       w.nchunk, w.wpart, pld);
   const int vw = pld % 4 == 0 && ((uintptr_t)a->grad & 15) == 0 ? 4 : 1;
   const int cblk = (int)((pld / vw + 63) / 64);
   HeadSum head{w.hpart, w.tile_rows == 64 ? (int)fgrid : 0, cblk, F.a_w3()};
