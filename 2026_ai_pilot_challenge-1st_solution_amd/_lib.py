@@ -206,12 +206,15 @@ class _LaunchStream:
 def launch_stream(device=None):
     """(stream, C handle) of the caller's current stream on `device`: every launch of this
     library goes there, and `record` marks its tensors as used on the same stream."""
-    index = device.index if isinstance(device, torch.device) else None
+    index = None
+    if device is not None:
+        if not isinstance(device, torch.device):
+            device = torch.device(device)
+        if device.type != "cuda":     # as torch.cuda.current_stream: no launch on host addresses
+            raise ValueError(f"a launch needs tensors on a GPU, not on {device}")
+        index = device.index
     if index is None:
-        if device is not None and not isinstance(device, torch.device):
-            index = torch.device(device).index
-        if index is None:
-            index = torch.cuda.current_device()
+        index = torch.cuda.current_device()
     h = torch._C._cuda_getCurrentRawStream(index)
     return _LaunchStream(h, index), ctypes.c_void_p(h)
 

@@ -64,6 +64,38 @@ def test_record_owned_follows_stream_and_buffer_objects():
     assert z.records == [2] and x.records == [1, 2]
 
 
+@pytest.mark.parametrize("device", ["cpu", "torch.device", "meta"])
+def test_launch_stream_refuses_a_device_without_streams(monkeypatch, device):
+    """Only a GPU device has a launch stream: any other is refused, as torch.cuda.current_stream
+    refuses it, before a launch could be handed its tensors' host addresses."""
+    import torch
+    L = import_pkg("_lib")
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0, raising=False)
+    assert L.launch_stream()[0].index == 0
+    assert L.launch_stream(torch.device("cuda", 1))[0].index == 1
+    with pytest.raises(ValueError):
+        L.launch_stream(torch.device("cpu") if device == "torch.device" else device)
+
+
+def test_host_tensors_are_not_launched(monkeypatch):
+    """gae and build_future_labels of CPU tensors raise before their entry points are called."""
+    import torch
+    L, R, F = import_pkg("_lib"), import_pkg("ppo"), import_pkg("future_aux")
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0, raising=False)
+    launched = []
+    entry = lambda *a: launched.append(a) or 0
+    monkeypatch.setattr(L, "lib", lambda: SimpleNamespace(f16_gae=entry,
+                                                          f16_future_labels=entry))
+    x = torch.zeros(3, 4)
+    with pytest.raises(ValueError):
+        R.gae(x, x, x, x[0], x[0])
+    with pytest.raises(ValueError):
+        F.build_future_labels(torch.zeros(3, 4, F.AUX_FEATURE_DIM, dtype=torch.float64), x, 0.1)
+    assert launched == []
+
+
 def _trace(env, initial, controls):
     """The reference's run_trace (kernel_stream_val.py:82-113): forced endings at steps 3 and
     7, every output, the states and the reconstructor per step."""
