@@ -190,17 +190,20 @@ def stream_handle(device=None):
 
 class _LaunchStream:
     """The caller's current stream on a device, by its raw handle; the torch.cuda.Stream object is
-    made only where a tensor has to be recorded (building one costs more than a launch)."""
-    __slots__ = ("cuda_stream", "index")
+    made only where a tensor has to be recorded (building one costs more than a launch), and then
+    once for all the launch's records."""
+    __slots__ = ("cuda_stream", "index", "_stream")
 
     def __init__(self, cuda_stream, index):
-        self.cuda_stream, self.index = cuda_stream, index
+        self.cuda_stream, self.index, self._stream = cuda_stream, index, None
 
     def torch_stream(self):
-        s = torch.cuda.current_stream(self.index)
-        if s.cuda_stream != self.cuda_stream:
-            raise RuntimeError("the current stream changed between a launch and its record")
-        return s
+        if self._stream is None:
+            s = torch.cuda.current_stream(self.index)
+            if s.cuda_stream != self.cuda_stream:
+                raise RuntimeError("the current stream changed between a launch and its record")
+            self._stream = s
+        return self._stream
 
 
 def launch_stream(device=None):

@@ -64,6 +64,31 @@ def test_record_owned_follows_stream_and_buffer_objects():
     assert z.records == [2] and x.records == [1, 2]
 
 
+def test_one_stream_object_per_launch(monkeypatch):
+    """A launch that has to record several groups of buffers (a new environment's first step) makes
+    one torch.cuda.Stream object for all of them, and none where every record is skipped."""
+    import torch
+    L = import_pkg("_lib")
+    made = []
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 77, raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream",
+                        lambda index: made.append(index) or SimpleNamespace(cuda_stream=77))
+    owners = [SimpleNamespace() for _ in range(3)]
+    bufs = [(_FakeTensor(0x100 * k), _FakeTensor(0x100 * k + 8)) for k in range(1, 5)]
+
+    def launch():
+        stream, _ = L.launch_stream()
+        for owner, b in zip(owners, bufs):
+            L.record_owned(owner, stream, b)
+        L.record(stream, bufs[3])
+
+    launch()
+    assert made == [0] and all(t.records == [77] for b in bufs for t in b)
+    launch()
+    assert made == [0] and all(t.records == [77] for b in bufs for t in b)
+
+
 @pytest.mark.parametrize("device", ["cpu", "torch.device", "meta"])
 def test_launch_stream_refuses_a_device_without_streams(monkeypatch, device):
     """Only a GPU device has a launch stream: any other is refused, as torch.cuda.current_stream
