@@ -428,8 +428,9 @@ class GpuDogfightVecEnv:
                 else None)
         terminal_hp = torch.empty(n, dtype=torch.float64, device=dev)
         terminal_alt = torch.empty(n, dtype=torch.float64, device=dev)
-        # one allocation for the four flags
-        term, trunc, done, fin = torch.empty(4, ne, dtype=torch.bool, device=dev).unbind()
+        # (a tensor each, as they are handed out: views of one would keep, save and version all four
+        # together, three of them off the allocator's alignment)
+        term, trunc, done, fin = (torch.empty(ne, dtype=torch.bool, device=dev) for _ in range(4))
         io = self._io(pick)
         self._call_tensors = (pick,)
         p = lambda t: t.data_ptr() if t is not None else None

@@ -695,6 +695,23 @@ def test_env_step_group_count_edges(gpu, obs_dim, nenv):
     assert resets > 0
 
 
+def test_step_flags_are_tensors_of_their_own(gpu):
+    """terminated, truncated, done and terminal_state_finite each own their memory, aligned as the
+    allocator aligns it: one kept or saved is not all four, and a word view of one works."""
+    E = import_pkg("rl_env").GpuDogfightVecEnv
+    nenv = 36
+    env = E(nenv, seed=3, ic_pool_size=16)
+    env.reset(stagger=False)
+    _, _, done, info = env.step(torch.zeros(2 * nenv, 4, dtype=torch.float64, device=gpu))
+    flags = [info["terminated"], info["truncated"], done, info["terminal_state_finite"]]
+    for t in flags:
+        assert t.shape == (nenv,) and t.dtype == torch.bool
+        assert t.untyped_storage().nbytes() == nenv and t.data_ptr() % 256 == 0
+        assert t.view(torch.int32).numel() == nenv // 4
+    assert len({t.untyped_storage().data_ptr() for t in flags}) == 4
+    assert info["done"] is done
+
+
 def test_step_training_and_capture_switch(gpu):
     """The root lineage's surface (cuda_fdm/rl_env.py:518-529): step_training and
     step(capture_terminal_obs=False) return the same observation, reward, done and info as a
