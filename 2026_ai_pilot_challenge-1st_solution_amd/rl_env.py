@@ -452,8 +452,12 @@ class GpuDogfightVecEnv:
     def norm_fuse_pays(self):
         """Whether a rollout's step is faster with the norm partials formed in its launch than
         with a separate RunningNorm.update: in a batch that gives 64-aircraft workgroups a compute
-        unit each the one-launch step uses those, which cannot form the 128-row partials."""
-        return not self.fused_step or bool(
+        unit each the one-launch step of four physics roles uses those, which cannot form the
+        128-row partials.  Every other step (two roles, or two launches) has 128 aircraft to a
+        workgroup in any batch."""
+        four_role = (self.fused_step and self.fused_finite and self.substeps >= 1
+                     and self.step_roles != 2)
+        return not four_role or bool(
             self.obr._lib.f16_env_step_norm_pays(self.nenv, self.OBS_SIZE))
 
     def step_rollout(self, reward_f32, done_f32, finite_acc, step_base=None, step=0, norm=None,
