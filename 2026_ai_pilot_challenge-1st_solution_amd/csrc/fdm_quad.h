@@ -102,8 +102,8 @@ enum QuadField : int {
   kQRho, kQSound, kQPres,                                // air
   kQMass, kQJ, kQJinv = kQJ + 6, kQRp = kQJinv + 6, kQCg = kQRp + 3,   // aero, parity block 0
   kQMassB = kQCg + 3,                                    // aero, parity block 1 (19 fields)
-  // after the last substep: each state-holding role's finite flag
-  kQFinKin = kQMassB + (kQMassB - kQMass), kQFinFcs,
+  // after the last substep: whether what each role stored is finite
+  kQFinKin = kQMassB + (kQMassB - kQMass), kQFinFcs, kQFinAero,
   // the kin role's own slots: values it reads once per substep, kept out of registers across the
   // phases that do not use them
   kQPba, kQPpd = kQPba + 3, kQPpq = kQPpd + 3,           // previous accelerations and rates
@@ -151,26 +151,6 @@ __device__ __forceinline__ void quad_kin(const Image& image, double* __restrict_
     sincos(a.epa + kRot * kDt, &se, &ce);
     x[kQCs][lane] = ce;
     x[kQCs + 1][lane] = se;
-  }
-  unsigned hist_m = 0u;   // as split_flight: only the entries shifted when S < 3 need a test
-  if (store && S > 0 && S < 3) {
-    for (int k = 2; k >= S; --k) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const double h = F(F16S_DQ + 4 * (k - S) + j);
-        hist_m = fin_acc(hist_m, h);
-        F(F16S_DQ + 4 * k + j) = h;
-      }
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const double h1 = F(F16S_DPQRI + 3 * (k - S) + j), h2 = F(F16S_DIVEL + 3 * (k - S) + j);
-        const double h3 = F(F16S_DUVW + 3 * (k - S) + j);
-        hist_m = fin_acc(fin_acc(fin_acc(hist_m, h1), h2), h3);
-        F(F16S_DPQRI + 3 * k + j) = h1;
-        F(F16S_DIVEL + 3 * k + j) = h2;
-        F(F16S_DUVW + 3 * k + j) = h3;
-      }
-    }
   }
   const bool out = out_base != nullptr && store;   // its part of the 17-value output
   for (int t = 0;; ++t) {
@@ -323,7 +303,7 @@ __device__ __forceinline__ void quad_kin(const Image& image, double* __restrict_
   }
 #undef F
   if (fin) {
-    unsigned m = fin_acc(hist_m, a.epa);
+    unsigned m = fin_acc(0u, a.epa);
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
       m = fin_acc(fin_acc(fin_acc(fin_acc(m, a.p[j]), a.v[j]), a.wi[j]), a.ai[j]);
@@ -337,11 +317,49 @@ __device__ __forceinline__ void quad_kin(const Image& image, double* __restrict_
 }
 
 // ---- aero: mass properties, and the six axes of the aero build-up but the lateral axes' late
-// terms.  Holds no state.
+// terms.  Holds no state, and in a step of one or two substeps shifts the history entries that
+// outlive it: all loaded at once while the other roles load their states, where the kin role
+// shifted them one entry after the other before its first pose (one substep of 64 / 16,384 /
+// 65,536 engagements: 12.05 / 15.9 / 59.2 -> 9.5 / 13.2 / 46.4 us; two: 14.0 / 18.5 / 64.7 ->
+// 12.2 / 16.6 / 58.0).
 template <int FCS_RATE, bool PRIO, class Image>
-__device__ __forceinline__ void quad_aero(const Image& image, int S, const double* __restrict__ T, QuadX& x,
-                                          int lane, bool fin) {
+__device__ __forceinline__ void quad_aero(const Image& image, double* __restrict__ s, long ld,
+                                          int S, bool store, const double* __restrict__ T,
+                                          QuadX& x, int lane, bool fin) {
   double vt = 0.0, vt2 = 0.0, alpha = 0.0, q = 0.0, lef = 0.0, flap = 0.0;
+  unsigned hist_m = 0u;   // as split_flight: only the entries shifted when S < 3 need a test
+  if (store && S > 0 && S < 3) {
+#define F(k) s[(long)(k) * ld]
+    double e[2][13];      // entries 0 and (S = 1) 1, which become S and 2
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (k > 0 && S == 2) break;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) e[k][j] = F(F16S_DQ + 4 * k + j);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        e[k][4 + j] = F(F16S_DPQRI + 3 * k + j);
+        e[k][7 + j] = F(F16S_DIVEL + 3 * k + j);
+        e[k][10 + j] = F(F16S_DUVW + 3 * k + j);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (k > 0 && S == 2) break;
+      const int to = k + S;
+#pragma unroll
+      for (int j = 0; j < 13; ++j) hist_m = fin_acc(hist_m, e[k][j]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) F(F16S_DQ + 4 * to + j) = e[k][j];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        F(F16S_DPQRI + 3 * to + j) = e[k][4 + j];
+        F(F16S_DIVEL + 3 * to + j) = e[k][7 + j];
+        F(F16S_DUVW + 3 * to + j) = e[k][10 + j];
+      }
+    }
+#undef F
+  }
   image.store();
   for (int t = 0;; ++t) {
     __syncthreads();
@@ -403,7 +421,10 @@ __device__ __forceinline__ void quad_aero(const Image& image, int S, const doubl
     }
   }
   quad_prio<0, PRIO>();
-  if (fin) __syncthreads();
+  if (fin) {
+    x[kQFinAero][lane] = hist_m < kFinInf ? 1.0 : 0.0;
+    __syncthreads();
+  }
 }
 
 // ---- fcs: the FCS channels, the previous-frame auxiliary values, and sin/cos of the Earth angle.
@@ -548,7 +569,7 @@ __device__ __forceinline__ void quad_fcs(const Image& image, double* __restrict_
 }
 
 // ---- air: atmosphere, engine and fuel.  With `fin` non-null, fin[0] <- 1 if all 101 state
-// values are finite (its own, and the kin and fcs roles' flags after the last barrier).
+// values are finite (its own, and the other roles' flags after the last barrier).
 template <int FCS_RATE, bool PRIO, class Image>
 __device__ __forceinline__ void quad_air(const Image& image, double* __restrict__ s, long ld,
                                          const double* __restrict__ act4, int S, bool store,
@@ -600,7 +621,8 @@ __device__ __forceinline__ void quad_air(const Image& image, double* __restrict_
     m = fin_acc(m, a.ff);
     __syncthreads();
     if (store)
-      fin[0] = (m < kFinInf && x[kQFinKin][lane] != 0.0 && x[kQFinFcs][lane] != 0.0) ? 1 : 0;
+      fin[0] = (m < kFinInf && x[kQFinKin][lane] != 0.0 && x[kQFinFcs][lane] != 0.0 &&
+                x[kQFinAero][lane] != 0.0) ? 1 : 0;
   }
 }
 
@@ -634,7 +656,7 @@ __global__ __launch_bounds__(256 * G) void fdm_step_quad_kernel(
     quad_kin<FCS_RATE, kPrio>(image, st + ia, ld, S, store, OBS ? obs + ia : nullptr, obs_ld, T, X[grp],
                               lane, fin != nullptr);
   else if (role == kRoleAero)
-    quad_aero<FCS_RATE, kPrio>(image, S, T, X[grp], lane, fin != nullptr);
+    quad_aero<FCS_RATE, kPrio>(image, st + ia, ld, S, store, T, X[grp], lane, fin != nullptr);
   else if (role == kRoleFcs)
     quad_fcs<FCS_RATE, kPrio>(image, st + ia, ld, act + 4L * ia, S, store, T, X[grp], lane,
                               fin != nullptr, act_keep ? act_keep + 4L * ia : nullptr,

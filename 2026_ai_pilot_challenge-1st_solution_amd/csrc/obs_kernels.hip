@@ -1589,7 +1589,7 @@ __global__ __launch_bounds__(256 * NG) void env_step_quad_kernel(const EnvStepAr
     f16::quad_kin<FCS_RATE, kPrio>(image, st, ld, S, store, nullptr, 0, L.fdm.T, L.fdm.X[grp],
                                    lane, true);
   else if (role == f16::kRoleAero)
-    f16::quad_aero<FCS_RATE, kPrio>(image, S, L.fdm.T, L.fdm.X[grp], lane, true);
+    f16::quad_aero<FCS_RATE, kPrio>(image, st, ld, S, store, L.fdm.T, L.fdm.X[grp], lane, true);
   else if (role == f16::kRoleFcs)
     f16::quad_fcs<FCS_RATE, kPrio>(image, st, ld, A.act + 4L * ia, S, store, L.fdm.T, L.fdm.X[grp],
                                    lane, true, A.act_keep ? A.act_keep + 4L * ia : nullptr);
