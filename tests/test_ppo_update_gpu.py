@@ -128,9 +128,12 @@ def test_minibatch_grad_matches_oracle(gpu, D, mb, ent_coef, norm_adv):
     assert float(stats[U_.STAT_BAD]) == 0.0
 
 
-@pytest.mark.parametrize("D,mb", [(184, 31), (214, 33), (184, 65), (214, 8191), (184, 8192),
-                                  (184, 8193), (214, 8257), (214, 20001)])
-def test_minibatch_grad_at_tile_edges(gpu, D, mb):
+@pytest.mark.parametrize("D,mb,norm_adv", [(184, 31, True), (214, 33, True), (184, 65, True),
+                                           (214, 8191, True), (184, 8192, True),
+                                           (184, 8193, True), (214, 8257, True),
+                                           (214, 20001, True), (214, 8200, False),
+                                           (184, 16449, False)])
+def test_minibatch_grad_at_tile_edges(gpu, D, mb, norm_adv):
     """Around the edges of the 32-row tiles (up to 8,192 rows on 256 compute units) and of the
     64-row tiles above, ragged and whole, with one and several tiles to a workgroup.  The tolerance
     is the smaller minibatches': the gradients differ from the bf16-mirrored oracle's only by fp32
@@ -138,17 +141,18 @@ def test_minibatch_grad_at_tile_edges(gpu, D, mb):
     row that such a rounding moves across one enters or leaves the sum of mb random rows, a
     relative change of about 1 / sqrt(mb) -- 7e-3 at 20,001 rows -- in either implementation."""
     U = import_pkg("ppo_update")
-    print(f"minibatch grad at tile edges D={D} mb={mb}", flush=True)
+    print(f"minibatch grad at tile edges D={D} mb={mb} norm_adv={norm_adv}", flush=True)
     net = make_net(D, seed=D + mb)
     flat = flat_of(net)
     ro, adv, ret = fake_rollout(flat, D, 1, mb + 7, seed=mb, logp_noise=0.0)
     pick = torch.randint(0, 4, (1, mb + 7), generator=torch.Generator().manual_seed(mb))
     ro.b_logp += torch.tensor([-0.4, -0.05, 0.05, 0.4])[pick]       # clip range: log 0.8, log 1.2
-    up = U.PPOUpdater(net.to(gpu), U.UpdateConfig(ent_coef=0.01))
+    up = U.PPOUpdater(net.to(gpu), U.UpdateConfig(ent_coef=0.01, norm_adv=norm_adv))
     idx = torch.randperm(mb + 7, generator=torch.Generator().manual_seed(7))[:mb]
     buf = [x.flatten(0, 1) for x in (ro.b_obs, ro.b_act, ro.b_logp, adv, ret)]
     up.minibatch_grad(*(x.to(gpu).contiguous() for x in buf), idx.to(gpu))
-    g_ref, st = P.mirror_minibatch(flat, D, *(x[idx] for x in buf), ent_coef=0.01)
+    g_ref, st = P.mirror_minibatch(flat, D, *(x[idx] for x in buf), ent_coef=0.01,
+                                   norm_adv=norm_adv)
     check_grads(up.grad.cpu(), g_ref, D, tol=3e-3)
     stats = up.stats[0].cpu()
     for k, j in (("pl", U.STAT_PL), ("vl", U.STAT_VL), ("ent", U.STAT_ENT), ("kl", U.STAT_KL)):
@@ -169,6 +173,55 @@ def test_out_of_range_indices_are_counted_not_read(gpu):
                       adv.reshape(-1).to(gpu), ret.reshape(-1).to(gpu), idx)
     assert float(up.stats[0, U.STAT_BAD]) == 3.0
     assert torch.isfinite(up.grad).all()
+
+
+@pytest.mark.parametrize("D,mb", [(184, 8300), (214, 16705)])
+def test_out_of_range_indices_in_several_tiles(gpu, D, mb):
+    """Bad indices in the first, a middle and the last 64-row tile (16,705 rows are 262 tiles, more
+    than one to some workgroups) are counted exactly and leave the other rows' gradient: the
+    oracle's of the good rows, whose means the minibatch's size divides.  The tolerance is four
+    times what bf16 roundings alone do to the first layer (1.6e-3 at 8,300 rows: the oracle against
+    itself with its parameters moved by 3e-7); one row too many or too few would be 1 / sqrt(mb),
+    7.7e-3 or more."""
+    U = import_pkg("ppo_update")
+    print(f"bad indices in several tiles D={D} mb={mb}", flush=True)
+    net = make_net(D, seed=11)
+    flat = flat_of(net)
+    ro, adv, ret = fake_rollout(flat, D, 1, mb, seed=4, logp_noise=0.0)
+    up = U.PPOUpdater(net.to(gpu), U.UpdateConfig(norm_adv=False))
+    good = torch.randperm(mb, generator=torch.Generator().manual_seed(3))
+    idx = good.clone()
+    last = (mb - 1) // 64 * 64
+    bad = [0, 1, 63, 64 * 70 + 5, 64 * 128, last, mb - 1]
+    for k, r in enumerate(bad):
+        idx[r] = (-1, mb, -2 ** 40, 2 ** 62)[k % 4]
+    keep = torch.ones(mb, dtype=torch.bool)
+    keep[bad] = False
+    buf = [x.flatten(0, 1) for x in (ro.b_obs, ro.b_act, ro.b_logp, adv, ret)]
+    up.minibatch_grad(*(x.to(gpu).contiguous() for x in buf), idx.to(gpu))
+    assert float(up.stats[0, U.STAT_BAD]) == len(set(bad))
+    g_ref, _ = P.mirror_minibatch(flat, D, *(x[good[keep]] for x in buf), norm_adv=False)
+    check_grads(up.grad.cpu(), g_ref * (int(keep.sum()) / mb), D, tol=6e-3)
+
+
+@pytest.mark.parametrize("mb", [300, 8300])
+def test_gradient_buffer_off_the_16_byte_grid(gpu, mb):
+    """A gradient buffer that is not 16-byte aligned takes the one-column sums: the same bits."""
+    U = import_pkg("ppo_update")
+    D = 184
+    net = make_net(D, seed=11)
+    ro, adv, ret = fake_rollout(flat_of(net), D, 1, mb, seed=4)
+    up = U.PPOUpdater(net.to(gpu))
+    args = [x.flatten(0, 1).to(gpu).contiguous()
+            for x in (ro.b_obs, ro.b_act, ro.b_logp, adv, ret)] + [torch.arange(mb, device=gpu)]
+    up.minibatch_grad(*args)
+    want, stats = up.grad.clone(), up.stats[0].clone()
+    hold = torch.full((up.grad.numel() + 2,), float("nan"), device=gpu)
+    up.grad = hold[1:-1]
+    assert want.data_ptr() % 16 == 0 and up.grad.data_ptr() % 16 == 4
+    up.minibatch_grad(*args)
+    assert torch.equal(up.grad, want) and torch.equal(up.stats[0], stats)
+    assert bool(hold[[0, -1]].isnan().all())
 
 
 def test_optimizer_step_matches_torch_adam(gpu):
@@ -212,26 +265,31 @@ def test_optimizer_step_writes_whole_blobs(gpu, D):
         assert torch.equal(g, b), name
 
 
-def test_update_matches_reference_loop(gpu):
-    """Two epochs of four minibatches (ragged last) with fixed permutations: final parameters,
-    statistics and norms against the reference loop with the mirrored gradients."""
+@pytest.mark.parametrize("rows,nmb,clip", [(130, 4, 0.2), (4199, 2, 10.0)])
+def test_update_matches_reference_loop(gpu, rows, nmb, clip):
+    """Two epochs of `nmb` minibatches with fixed permutations -- of 130 rows, and of 8,398, which
+    take the 64-row tiles -- final parameters, statistics and norms against the reference loop with
+    the mirrored gradients.  The larger minibatches are not clipped: of their rows, about one in a
+    thousand has a ratio so close to a clip's edge that a bf16 rounding moves it across, each such
+    row changes the gradient by 1 / sqrt(8,398) of its norm, 1.1 %, and Adam's first steps then
+    differ by 5 % in every coordinate below 0.2 of the gradient's spread."""
     U = import_pkg("ppo_update")
     D = 184
     net = make_net(D, seed=21)
     flat = flat_of(net)
-    T, rows = 4, 130
+    T = 4
     ro, adv, ret = fake_rollout(flat, D, T, rows, seed=22, logp_noise=0.05)
     count = T * rows
     gen = torch.Generator().manual_seed(23)
     perms = [torch.randperm(count, generator=gen) for _ in range(2)]
-    cfg = U.UpdateConfig(update_epochs=2, num_minibatches=4, target_kl=None)
+    cfg = U.UpdateConfig(update_epochs=2, num_minibatches=nmb, target_kl=None, clip_coef=clip)
     up = U.PPOUpdater(net.to(gpu), cfg)
     res = up.update(to_dev(ro, gpu), adv.to(gpu), ret.to(gpu), perms=perms)
-    mb = (count + 3) // 4
+    mb = (count + nmb - 1) // nmb
     p_ref, rr = P.reference_update(flat, D, ro.b_obs.flatten(0, 1), ro.b_act.flatten(0, 1),
                                    ro.b_logp.flatten(), adv.reshape(-1), ret.reshape(-1), perms,
-                                   mb, target_kl=None)
-    assert res["optimizer_steps"] == rr["optimizer_steps"] == 8
+                                   mb, clip=clip, target_kl=None)
+    assert res["optimizer_steps"] == rr["optimizer_steps"] == 2 * nmb
     assert res["epochs"] == 2 and not res["early"]
     p_gpu = up.flat.cpu()
     diff = (p_gpu - p_ref).abs()
@@ -242,7 +300,7 @@ def test_update_matches_reference_loop(gpu):
     # gradient difference e (bf16 rounding flips and accumulation order, ~1e-3) moves it by about
     # e * lr per step, and an element near zero can change sign: bound the worst by the steps'
     # total, the typical coordinate by 1 % of one step, and the far tail by its share
-    lr, steps = cfg.lr, 8
+    lr, steps = cfg.lr, 2 * nmb
     far = float((diff > 0.05 * lr).float().mean())
     print("  share of coordinates off by more than 5 %% of a step: %.2e" % far, flush=True)
     assert float(diff.max()) <= 2 * lr * steps
@@ -278,13 +336,14 @@ def test_early_stop_and_refusals(gpu):
         up.update(to_dev(ro, gpu), adv[:1].to(gpu), ret.to(gpu))
 
 
-def test_first_minibatch_of_a_rollout_has_ratio_one(gpu):
+@pytest.mark.parametrize("nenv", [64, 1040])     # 1,024 rows; 16,640: 64-row tiles, some twice
+def test_first_minibatch_of_a_rollout_has_ratio_one(gpu, nenv):
     """At the collection weights the update's log-probability equals the rollout kernel's bit
     for bit: every ratio is exactly 1, so the approximate KL and the clip fraction are 0."""
     ppo = import_pkg("ppo")
     U = import_pkg("ppo_update")
     rl = import_pkg("rl_env")
-    env = rl.GpuDogfightVecEnv(64, seed=0, ic_pool_size=64)
+    env = rl.GpuDogfightVecEnv(nenv, seed=0, ic_pool_size=64)
     net = make_net(184, seed=41).to(gpu)
     ro = ppo.SelfPlayRollout(env, net, T=8, seed=3, stats=False)
     ro.reset(stagger=True, max_stagger_steps=8)
@@ -455,14 +514,14 @@ def test_epoch_advantage_stats_equal_per_minibatch(gpu):
     D = 184
     net = make_net(D, seed=11)
     flat = flat_of(net)
-    T, rows = 7, 1000
+    T, rows = 7, 2500
     ro, adv, ret = fake_rollout(flat, D, T, rows, seed=3)
     up = U.PPOUpdater(net.to(gpu), U.UpdateConfig())
     d = to_dev(ro, gpu)
     obs, act, logp = d.b_obs.flatten(0, 1), d.b_act.flatten(0, 1), d.b_logp.flatten()
     advd, retd = adv.reshape(-1).to(gpu), ret.reshape(-1).to(gpu)
     count = T * rows
-    for mb in (2048, 2049, 1000, 333, count):
+    for mb in (2048, 2049, 1000, 333, 8193, count):      # (17,500 rows are 274 64-row tiles)
         perm = torch.randperm(count, generator=torch.Generator().manual_seed(mb)).to(gpu)
         st = up.epoch_adv_stats(advd, perm, mb)
         nmb = (count + mb - 1) // mb
@@ -483,9 +542,9 @@ def test_epoch_advantage_stats_equal_per_minibatch(gpu):
     work = torch.empty(1 << 20, dtype=torch.uint8, device=gpu)
     args = lambda total, mb, nmb: lib.f16_ppo_adv_stats(L.ptr(advd), L.ptr(perm), total, count,
                                                         mb, nmb, L.ptr(out), L.ptr(work), h)
-    assert args(count, 1000, 7) == 0
+    assert args(count, 2500, 7) == 0
     torch.cuda.synchronize()
-    assert args(count, 1000, 6) == L.F16_EINVAL      # too few minibatches for the cut
-    assert args(count, 1000, 8) == L.F16_EINVAL      # one minibatch past the end
+    assert args(count, 2500, 6) == L.F16_EINVAL      # too few minibatches for the cut
+    assert args(count, 2500, 8) == L.F16_EINVAL      # one minibatch past the end
     assert args(0, 1000, 1) == L.F16_EINVAL
     assert lib.f16_ppo_adv_work_bytes(0, 1) == -1

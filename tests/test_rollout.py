@@ -159,19 +159,36 @@ def test_graph_league_rollout_equals_eager(gpu):
     assert a.b_done.sum().item() > 0          # autoresets and opponent redraws happened
 
 
-@pytest.mark.parametrize("nenv,graph", [(200, False), (512, True)])
-def test_fused_norm_partials_equal_separate_update(gpu, nenv, graph):
+@pytest.mark.parametrize("nenv,graph,roles", [(200, False, None), (512, True, None),
+                                              (300, False, 2), (8201, False, 4), (8201, True, 4)])
+def test_fused_norm_partials_equal_separate_update(gpu, monkeypatch, nenv, graph, roles):
     """The post-physics launch forming the RunningNorm partial sums of the rows the next step
     normalises (then only the merge runs) gives the same statistics and buffers, bit for bit, as
     a separate f16_norm_update per step: over three rollouts with autoresets, a ragged last
-    128-row block (nenv 200) and the fused collector recorded as a HIP graph."""
+    128-row block (nenv 200, 300 and 8,201) and the fused collector recorded as a HIP graph.  At
+    8,201 engagements, and with two physics roles, the collector takes the fused sums by itself;
+    where its step's 64-aircraft workgroups make them a loss (`roles` None) they are asked for."""
     short = {"max_engage_time_s": 1.5}          # every engagement ends within 15 decisions
     a = _collector(gpu, nenv=nenv, T=8, stats=False, fuse_norm=False, env_kw=short)
     b = _collector(gpu, nenv=nenv, T=8, stats=False, graph=graph, fuse_norm=True, env_kw=short)
     assert not a.fuse_norm and b.fuse_norm
+    if roles is None:
+        assert not b.env.norm_fuse_pays()
+        monkeypatch.setattr(b.env, "norm_fuse_pays", lambda: True)
+    else:
+        a.env.step_roles = b.env.step_roles = roles
+        assert b.env.norm_fuse_pays()
+    calls = {}
+    for ro in (a, b):
+        for name in ("merge", "update"):
+            monkeypatch.setattr(ro.norm, name, lambda *x, ro=ro, name=name, fn=getattr(
+                ro.norm, name), **kw: (calls.update({(ro is b, name): calls.get(
+                    (ro is b, name), 0) + 1}), fn(*x, **kw))[1])
     done = 0.0
     for r in range(3):
         ra, rb = a.collect(), b.collect()
+        if r == 0:                             # (a graph's replays make no calls)
+            assert calls == {(False, "update"): a.T, (True, "update"): 1, (True, "merge"): b.T - 1}
         torch.cuda.synchronize()
         for name in BUFFERS:
             assert torch.equal(getattr(a, name), getattr(b, name)), (r, name)
