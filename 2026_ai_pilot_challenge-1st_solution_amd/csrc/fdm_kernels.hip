@@ -245,9 +245,10 @@ static int fdm_step_split(double* states, long ld, const double* actions, int na
                           int fcs_rate, double* obs, long obs_ld, unsigned char* fin,
                           void* stream, double* keep = nullptr, bool quad = true) {
   hipStream_t s = (hipStream_t)stream;
-  // The four-wave kernel (16k tail-chase engagements: 32.8 vs 36.7 us without the 17-value
-  // output, 36.3 vs 37.8 us with it; 64k: 133 vs 144 us, 142 vs 147 us).  Two groups per
-  // workgroup once the batch gives every CU such a workgroup, else one group per workgroup.
+  // The four-wave kernel (16k tail-chase engagements: 31.0 us against the two-wave kernel's 37.0
+  // without the 17-value output, 32.4 against 38.7 with it; 64k: 110 against 140 us, 115 against
+  // 145).  Two groups per workgroup once the batch gives every CU such a workgroup, else one group
+  // per workgroup.
   if (quad) {
     const bool two = (long)nac >= (long)f16::kQuadAircraft * device_cus();
 #define F16_QUAD(R, O, G)                                                                     \

@@ -5,7 +5,8 @@
 // such groups, or one in a small batch):
 //   kin   the integrator: pose and motion, frames, gravity, forces, moments, accelerations, and
 //         the late (Mach) terms of the side, roll and yaw axes;
-//   aero  mass properties and the rest of the aero build-up;
+//   aero  mass properties, the rest of the aero build-up, and the history shift of a step of one
+//         or two substeps;
 //   fcs   the flight control system, the previous-frame auxiliary values, sin/cos of the Earth
 //         angle and, after the last substep, most of the 17-value output;
 //   air   atmosphere, engine, fuel.
@@ -26,11 +27,11 @@
 // kernel took 1.6, 1.25 and 1.3: a lone wavefront issues one instruction every 4-5 clocks,
 // VALU or not (fp64 included, no extra latency when dependent), so a window costs the longest
 // role's instruction count and the split is chosen to make those equal.  Measured per step
-// (tail-chase, HIP-graph replay, before -> after): 2,048 engagements 26.3 -> 23.6 us, 64 with the
-// 17-value output 28.7 -> 24.3, 16,384 with it 33.6 -> 30.7 and without 29.8 -> 29.7 (there two
-// wavefronts share each SIMD and the VALU is the bound), 65,536 115 -> 112; the single-precision
-// build 16,384 26.3 -> 22.6, 64 24.5 -> 20.7.  The env step at 16,384 engagements 65.3 -> 59.1 us
-// (of which the supersonic passes left to the last substep 3.4).
+// (tail-chase, HIP-graph replay), four roles in that order and in this one: 2,048 engagements 26.5 -> 24.0 us,
+// 64 with the 17-value output 28.0 -> 24.3, 16,384 with it 35.9 -> 32.4 and without 32.4 -> 31.0
+// (there two wavefronts share each SIMD), 65,536 115 -> 110; the single-precision build 16,384
+// 26.0 -> 22.1, 64 23.8 -> 19.1.  The env step at 16,384 engagements 59.9 -> 52.9 us (of which the
+// supersonic passes left to the last substep 3.4).
 //
 // Every value is formed by the component functions of fdm_device.h with the operands the
 // one-lane kernel gives them, so all three kernels agree bit for bit.  An aero axis is summed

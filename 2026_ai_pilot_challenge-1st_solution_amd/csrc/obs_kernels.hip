@@ -1545,7 +1545,8 @@ __global__ __launch_bounds__(kPostSplitBlock) void env_step_fused_kernel(
 // The same step with each 64 aircraft on four wavefronts in both phases (fdm_quad.h's four physics
 // roles, then post_quad_body's four post-physics roles).  NG = 2 (512-thread workgroups): at
 // 16,384 engagements every SIMD holds two wavefronts instead of one.  NG = 1: a small batch
-// spreads over twice the CUs, one wavefront per SIMD, so neither phase shares its issue slots.  Results equal env_step_fused_kernel's bit for bit.
+// spreads over twice the CUs, one wavefront per SIMD, so neither phase shares its issue slots.
+// Results equal env_step_fused_kernel's bit for bit.
 template <int D, int NG>
 union EnvQuadLds {
   struct {
@@ -1703,10 +1704,13 @@ static bool full_tile_resident(int nenv, int obs_dim, int groups = 1) {
 }
 
 // Whether the one-launch step takes one 64-aircraft group per workgroup: while every such
-// workgroup has a CU of its own (8,192 engagements on 256 CUs).  Rollout of 64 steps at 200 /
-// 4,000 / 9,000 / 15,000 engagements with two groups per workgroup and with one: 4.34 / 4.78 /
-// 5.69 / 5.91 ms and 3.97 / 4.43 / 5.64 / 6.14 ms, the latter with the norm's partial sums in a
-// launch of their own; a league of 2,000 and 12,000 (32 steps): 6.15, 3.39 and 5.63, 3.42 ms.
+// workgroup has a CU of its own (8,192 engagements on 256 CUs).  With two groups per workgroup and
+// with one: the env step at 214 columns of 777 / 4,000 / 8,192 engagements 52.7 / 54.5 / 56.9 and
+// 50 / 49.6 / 50 us; a self-play rollout of 32 steps (the norm's partial sums in a launch of their
+// own with one group) of 200 / 4,000 / 8,192 engagements 2.18 / 2.37 / 2.63 and 1.99 / 2.19 /
+// 2.51 ms, a league's of 2,000 and 8,192 2.98, 3.30 and 2.72, 3.08 ms.  Beyond the line two
+// workgroups share a CU: the rollout of 8,193 / 9,000 / 10,000 / 12,288 engagements takes 2.79 /
+// 2.88 / 2.89 / 2.94 and 2.69 / 2.86 / 2.91 / 2.99 ms.
 static bool env_step_one_group(int nenv) {
   return 2L * nenv <= (long)kRowBlock * resident_device().cus;
 }

@@ -56,7 +56,7 @@ struct Flat {
   __host__ __device__ long a_b1() const { return 256 * D; }
   __host__ __device__ long a_w2() const { return 256 * D + 256; }
   __host__ __device__ long a_b2() const { return 256 * D + 65792; }
-  __host__ __device__ long a_w3() const { return 256 * D + 66048; }
+  __host__ __device__ constexpr long a_w3() const { return 256 * D + 66048; }
   __host__ __device__ long a_b3() const { return 256 * D + 87552; }
   __host__ __device__ long na() const { return 256 * D + 87636; }
   __host__ __device__ long c_w1() const { return na(); }
@@ -84,7 +84,7 @@ constexpr int kFusedWG = 256;                    // bound on the fused kernel's 
 __host__ __device__ inline long align256(long x) { return (x + 255) & ~255L; }
 
 struct Work {
-  float* advs;          // [8]: mean, std, statistics sums
+  float* advs;          // [2]: the advantages' mean and std
   double* normp;        // [nblk][2] squared-norm partials
   __bf16 *xt, *h1t, *h2t, *dh1t, *dh2t, *dzt;   // unit-major in 64-row blocks (ublock); features
                                                 // kp, 512, 256, 512, 512, kLogitsPad
@@ -982,11 +982,15 @@ __global__ __launch_bounds__(kThreads, 1) void ppo_fused_kernel(const F16PPOArgs
 }
 
 // ---- weight gradients: C[a][b] = sum over rows of A[a][row] B[b][row], split over row chunks.
-// Output tiles are 256 x 256, so each product's operands are read once per row chunk (the
-// first layer's input twice, beside the two 256-unit halves of dH1): the kernel streams ~4.5 KB
-// per minibatch row against 4.2 KB of distinct operands.  Eight waves, 2 (A halves of 128) x 4
-// (B quarters of 64), each accumulating a 128 x 64 block as 4 x 2 MFMA 32x32 tiles; 64-row
-// stages double-buffered through LDS (147 KB), one workgroup per CU.
+// Two forms, with TA features of A by 256 of B to a tile; eight waves, 2 (A halves) x 4 (B quarters
+// of 64), 64-row stages double-buffered through LDS, one workgroup per CU:
+//   TA = 256  each wave accumulates 128 x 64 as 4 x 2 MFMA 32x32 tiles; 147 KB of LDS.  Each
+//             product's operands are read once per row chunk, the first layer's input twice
+//             (beside the two 256-unit halves of dH1).  At 184 columns, per minibatch row: 3.8 KB
+//             streamed of 3.5 KB of distinct operands with 64-row tiles (the first and the two
+//             second layers, four tiles), 4.5 of 4.2 with 32-row tiles (the actor's head too, five);
+//   TA = 128  (small minibatches: f16_ppo_grad) 64 x 64 to a wave, 111 KB of LDS, nine tiles; the
+//             layer input is read four times and the second layers' twice.
 constexpr int kWT = 256;                  // output tile side
 constexpr int kWK = 64;                   // rows per stage
 constexpr int kWPitch = kWK + 8;          // bf16 per LDS feature row (16-byte aligned, spread over banks)
@@ -1223,7 +1227,9 @@ __device__ __forceinline__ void tail_colsum(const TailSum& T, int blk) {
 
 // The actor head's partials (64-row tiles): the last blocks of a column-sum launch add them over
 // the fused kernel's workgroups, VW columns to a thread, 16 row phases combined in order, and the
-// other blocks leave the head's columns alone (kHead3 and its offset are multiples of 4).
+// other blocks leave the head's columns alone.
+static_assert(kHead3 % 4 == 0 && Flat{184}.a_w3() % 4 == 0 && Flat{214}.a_w3() % 4 == 0,
+              "the head is a whole number of 4-column groups of the flat parameters");
 struct HeadSum {
   const float* part;    // [nrows][kHead3]
   int nrows;            // 0: the head is among the other columns
@@ -1695,9 +1701,11 @@ static int wgrad_slots() {
 }
 
 // Rows of a fused-kernel tile.  While 32-row tiles find a CU each, half the work per tile ends
-// sooner (5,000 rows: a minibatch and its optimizer step 86.0 -> 77.0 us); with more of them the
-// weights' stream, the same for a tile of either size, costs more (262,144 rows in 32-row tiles,
-// two workgroups a CU: fused kernel 0.66 ms against 0.50).
+// sooner; with more of them the weights' stream, the same for a tile of either size, costs more.
+// Gradient and optimizer step at 184 / 214 columns in 32-row and in 64-row tiles: 5,000 rows 57.3 /
+// 58.3 and 66.8 / 67.3 us, 8,192 (the last with 32 on 256 CUs) 67.2 / 69.3 and 73.0 / 74.4, 8,193
+// 83.3 / 84.8 and 77.0 / 78.3, 12,288 86.9 / 90.2 and 83.0 / 86.2, 16,384 91 / 95 and 93 / 99;
+// 262,144 rows, the kernel alone with two workgroups a CU, 0.66 and 0.50 ms.
 static int fused_tile_rows(long mb_rows) {
   const long tiles = (mb_rows + 63) / 64 * 2;
   return tiles <= std::min(device_cus(), kFusedWG) ? 32 : 64;
@@ -1741,7 +1749,8 @@ extern "C" int f16_ppo_grad(const F16PPOArgs* a, void* stream) {
     hipLaunchKernelGGL((ppo_fused_kernel<224, 64>), dim3(fgrid), dim3(kThreads), 0, s, *a, w);
   else
     hipLaunchKernelGGL((ppo_fused_kernel<224, 32>), dim3(fgrid), dim3(kThreads), 0, s, *a, w);
-  // the four weight-gradient products and their tiles
+  // the weight-gradient products and their tiles: the first layers (one product), the two second
+  // layers and, with 32-row tiles, the actor's head
   WJobs J{};
   const long na = F.na();
   constexpr long kB512 = 512 * kUBlock, kB256 = 256 * kUBlock;
@@ -1758,8 +1767,11 @@ extern "C" int f16_ppo_grad(const F16PPOArgs* a, void* stream) {
   const int njob = w.tile_rows == 32 ? 4 : 3;   // else the fused kernel summed the head's
   int nt = 0;
   // Halves of the 256-feature A side while they too find a CU each: a stage is bound by the bytes
-  // a CU streams, and half a tile has 48 KB of 64 and half the results to write (5,000 rows: 22.0 -> 16.0 us).
-  // In a larger minibatch B's second reading costs more than the idle CUs.
+  // a CU streams, and half a tile has 48 KB of 64 and half the results to write.  In a larger
+  // minibatch B's second reading costs more than the idle CUs.  Gradient and optimizer step at 184 /
+  // 214 columns, halves and whole tiles: 5,000 rows 57.3 / 58.3 and 63.6 / 64.4 us, 7,168 (the last
+  // with halves on 256 CUs) 60.8 / 63.3 and 65.7 / 68.0, 7,169 69.3 / 70.4 and 66.3 / 67.0, 16,384
+  // 101 / 104 and 93 / 99.
   const int ntile128 = 8 + (njob == 4 ? 1 : 0);
   const int TA = ntile128 * w.nchunk <= wgrad_slots() ? 128 : kWT;
   int ntA[4], ntB[4];
