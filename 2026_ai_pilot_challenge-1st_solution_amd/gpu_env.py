@@ -148,7 +148,11 @@ class GpuDogfight:
         reference copies the actions into self.actions before its launch; a separate contiguous
         device tensor is returned as is (the launch reads it and writes the copy itself),
         anything else is copied into self.actions here and self.actions is returned."""
-        a = torch.as_tensor(actions, dtype=self.dtype, device=self.device).reshape(self.nac, 4)
+        return self._action_source(
+            torch.as_tensor(actions, dtype=self.dtype, device=self.device).reshape(self.nac, 4))
+
+    def _action_source(self, a):
+        """action_source of a (nac, 4) tensor of this simulator's dtype and device."""
         if self.precision == "fp64" and (a.is_contiguous() and a.untyped_storage().data_ptr()
                 != self.actions.untyped_storage().data_ptr()):
             return a

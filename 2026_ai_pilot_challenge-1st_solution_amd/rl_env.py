@@ -330,7 +330,8 @@ class GpuDogfightVecEnv:
         return io
 
     def _advance(self, io, actions, state_fin):
-        """The physics step of `actions` and the post-physics step `io` describes: one
+        """The physics step of `actions` (float64 (nac, 4) on the device) and the post-physics step
+        `io` describes: one
         f16_env_step launch with fused_step and the finite flags (state_fin) on (where the
         batch exceeds what the full-row tile keeps resident it issues the two launches itself),
         else sim.step and f16_env_post_step.  kernel_events, when a list, gets the one launch's
@@ -340,7 +341,7 @@ class GpuDogfightVecEnv:
             io.state_finite = state_fin.data_ptr() if state_fin is not None else None
             self._post(io)
             return
-        a = self.sim.action_source(actions)
+        a = self.sim._action_source(actions)
         io.state_finite = state_fin.data_ptr()
         c = self._cfg_struct()
         ev = self.kernel_events
@@ -376,13 +377,14 @@ class GpuDogfightVecEnv:
         self._post_steps += 1
 
     def _cfg_struct(self):
-        key = (tuple(sorted(self.reward_cfg.items())), self.min_altitude_m, self.max_engage_time_s,
-               self.reward_mode, self.alt_hunt_coef, self.fuel_exhaustion)
-        if self._cfg_key != key:
+        # (the configuration compared as a dict: sorted into a tuple on every step it cost 1.6 us)
+        key = (self.min_altitude_m, self.max_engage_time_s, self.reward_mode, self.alt_hunt_coef,
+               self.fuel_exhaustion)
+        if self._cfg_key is None or self._cfg_key[0] != self.reward_cfg or self._cfg_key[1] != key:
             self._cfg = reward_cfg_struct(self.reward_cfg, self.min_altitude_m,
                                           self.max_engage_time_s, self.reward_mode,
                                           self.alt_hunt_coef, self.fuel_exhaustion)
-            self._cfg_key = key
+            self._cfg_key = (dict(self.reward_cfg), key)
         return self._cfg
 
     def step_training(self, actions):
@@ -426,17 +428,18 @@ class GpuDogfightVecEnv:
         reward = torch.empty(n, dtype=torch.float64, device=dev)
         tobs = (torch.empty(n, self.OBS_SIZE, dtype=torch.float32, device=dev) if terminal_obs
                 else None)
-        terminal_hp = torch.empty(n, dtype=torch.float64, device=dev)
-        terminal_alt = torch.empty(n, dtype=torch.float64, device=dev)
+        terminal_hp, terminal_alt = torch.empty_like(reward), torch.empty_like(reward)
         # (a tensor each, as they are handed out: views of one would keep, save and version all four
         # together, three of them off the allocator's alignment)
-        term, trunc, done, fin = (torch.empty(ne, dtype=torch.bool, device=dev) for _ in range(4))
+        term = torch.empty(ne, dtype=torch.bool, device=dev)
+        trunc, done, fin = torch.empty_like(term), torch.empty_like(term), torch.empty_like(term)
         io = self._io(pick)
         self._call_tensors = (pick,)
-        p = lambda t: t.data_ptr() if t is not None else None
-        io.terminal_obs, io.reward = p(tobs), p(reward)
-        io.term, io.trunc, io.done, io.terminal_finite = p(term), p(trunc), p(done), p(fin)
-        io.terminal_hp, io.terminal_alt_m = p(terminal_hp), p(terminal_alt)
+        io.terminal_obs = tobs.data_ptr() if tobs is not None else None
+        io.reward = reward.data_ptr()
+        io.term, io.trunc = term.data_ptr(), trunc.data_ptr()
+        io.done, io.terminal_finite = done.data_ptr(), fin.data_ptr()
+        io.terminal_hp, io.terminal_alt_m = terminal_hp.data_ptr(), terminal_alt.data_ptr()
         self._advance(io, a, state_fin)
         info = {"terminated": term, "truncated": trunc,
                 "terminal_obs": tobs.view(ne, 2, self.OBS_SIZE) if tobs is not None else None,
