@@ -3,17 +3,17 @@
 //
 // The model is the fp64 one, not a second copy: build.py writes float copies of the model
 // headers (fdm_quad.h, fdm_split.h, fdm_advance.h, fdm_device.h, fdm_image.h, f16_model_gen.h,
-// f16_state.h, the generated tables) under _build/f32/ -- every double made float, every floating literal given an f suffix,
-// the libm calls made their float forms, namespace f16 renamed f16f -- and this file includes
-// those copies.  The reference derives its fp32 build from its fp64 source the same way
+// f16_state.h, the generated tables) under _build/f32/ -- every double made float, every floating
+// literal given an f suffix, the libm calls made their float forms, namespace f16 renamed f16f --
+// and this file includes those copies.  The reference derives its fp32 build from its fp64 source the same way
 // (cuda_rt.to_fp32, cuda_fdm/tests/cuda_rt.py:150-160).
 //
 // The kernel is fdm_quad.h's four-role form, each 64 aircraft on four cooperating wavefronts
-// (92-100 registers a lane in float: up to five wavefronts per SIMD).  Measured at 16,384
-// tail-chase engagements, 6 substeps, HIP events around each launch: 27.9 us against 36.6 us
-// for the fp64 build and 48.5 us for one lane per aircraft doing the whole substep in float
-// (316 registers a lane, one wavefront per SIMD, and half the SIMDs without one: the same
-// results bit for bit); at 65,536 engagements 66.5 us against 133 us in fp64.
+// (98-108 registers a lane in float: four wavefronts per SIMD).  Measured per step at 16,384
+// tail-chase engagements, 6 substeps (HIP-graph replay): 22.1 us against 31.0 us for the fp64
+// build; one lane per aircraft doing the whole substep in float (316 registers a lane, one
+// wavefront per SIMD, and half the SIMDs without one: the same results bit for bit) took 48.5;
+// at 65,536 engagements 56 us against 110 us in fp64.
 // Layout as in fdm_kernels.hip: field k of aircraft a at states[k * ld + a], output (17, obs_ld).
 #include <hip/hip_runtime.h>
 

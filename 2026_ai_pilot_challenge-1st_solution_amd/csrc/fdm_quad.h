@@ -27,11 +27,12 @@
 // kernel took 1.6, 1.25 and 1.3: a lone wavefront issues one instruction every 4-5 clocks,
 // VALU or not (fp64 included, no extra latency when dependent), so a window costs the longest
 // role's instruction count and the split is chosen to make those equal.  Measured per step
-// (tail-chase, HIP-graph replay), four roles in that order and in this one: 2,048 engagements 26.5 -> 24.0 us,
-// 64 with the 17-value output 28.0 -> 24.3, 16,384 with it 35.9 -> 32.4 and without 32.4 -> 31.0
-// (there two wavefronts share each SIMD), 65,536 115 -> 110; the single-precision build 16,384
-// 26.0 -> 22.1, 64 23.8 -> 19.1.  The env step at 16,384 engagements 59.9 -> 52.9 us (of which the
-// supersonic passes left to the last substep 3.4).
+// (tail-chase, HIP-graph replay), four roles in that order and in this one: 2,048 engagements
+// 26.5 -> 24.0 us, 64 with the 17-value output 28.0 -> 24.3, 16,384 with it 35.9 -> 32.4 and
+// without 32.4 -> 31.0 (there two wavefronts share each SIMD and issue during 75 % of its time),
+// 65,536 115 -> 110; the single-precision build 16,384 26.0 -> 22.1, 64 23.8 -> 19.1.  The env step
+// at 16,384 engagements 59.9 -> 52.9 us (of which the supersonic passes left to the last substep
+// 3.4).
 //
 // Every value is formed by the component functions of fdm_device.h with the operands the
 // one-lane kernel gives them, so all three kernels agree bit for bit.  An aero axis is summed
