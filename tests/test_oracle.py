@@ -91,7 +91,7 @@ def _py_literal(path, name):
     raise KeyError(name)
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference checkout absent")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REF, "cuda_fdm")), reason="reference checkout absent")
 def test_model_image_matches_reference_data(orc):
     """Our XML parser's tables equal the numbers in the reference's extracted data (read as
     text: cuda_fdm/ref/f16_aero_data.py, jsb_propulsion.py)."""
@@ -124,7 +124,7 @@ def test_model_image_matches_reference_data(orc):
         assert list(img[off:off + len(flat)]) == flat, tname
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference checkout absent")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REF, "cuda_fdm")), reason="reference checkout absent")
 def test_derived_constants_match_reference_header():
     """Start-up constants equal the values printed in cuda_fdm/gen/f16_gen.cuh:9-60."""
     txt = open(os.path.join(REF, "cuda_fdm/gen/f16_gen.cuh"), encoding="utf-8").read()
