@@ -497,7 +497,8 @@ template <int ROWS>
 __device__ __forceinline__ long long idx_load(const F16PPOArgs& a, int t, int tid) {
   long long p = kNoRow;
   const long r = (long)t * ROWS + tid;
-  if (tid < ROWS && r < a.mb_rows) p = a.idx[r];
+  // (an index of kNoRow, or below, is a bad one like any other)
+  if (tid < ROWS && r < a.mb_rows) p = max(a.idx[r], kNoRow + 1);
   return p;
 }
 template <int ROWS>

@@ -194,7 +194,7 @@ def test_out_of_range_indices_in_several_tiles(gpu, D, mb):
     last = (mb - 1) // 64 * 64
     bad = [0, 1, 63, 64 * 70 + 5, 64 * 128, last, mb - 1]
     for k, r in enumerate(bad):
-        idx[r] = (-1, mb, -2 ** 40, 2 ** 62)[k % 4]
+        idx[r] = (-1, mb, -2 ** 62, 2 ** 62, -2 ** 63)[k % 5]
     keep = torch.ones(mb, dtype=torch.bool)
     keep[bad] = False
     buf = [x.flatten(0, 1) for x in (ro.b_obs, ro.b_act, ro.b_logp, adv, ret)]
