@@ -207,22 +207,22 @@ class _LaunchStream:
         return s
 
 
-_gpu_index = {}      # GPU torch.device with an index -> that index (its type costs 0.2 us to read)
+# GPU devices as callers name them -> their index, or _CURRENT where they name none (None, "cuda"):
+# reading a torch.device's type costs 0.2 us
+_CURRENT = -1
+_gpu_index = {None: _CURRENT}
 
 
 def launch_stream(device=None):
     """(stream, C handle) of the caller's current stream on `device`: every launch of this
     library goes there, and `record` marks its tensors as used on the same stream."""
     index = _gpu_index.get(device)
-    if index is None and device is not None:
-        if not isinstance(device, torch.device):
-            device = torch.device(device)
-        if device.type != "cuda":     # as torch.cuda.current_stream: no launch on host addresses
-            raise ValueError(f"a launch needs tensors on a GPU, not on {device}")
-        index = device.index
-        if index is not None:
-            _gpu_index[device] = index
     if index is None:
+        d = device if isinstance(device, torch.device) else torch.device(device)
+        if d.type != "cuda":     # as torch.cuda.current_stream: no launch on host addresses
+            raise ValueError(f"a launch needs tensors on a GPU, not on {d}")
+        index = _gpu_index[device] = _CURRENT if d.index is None else d.index
+    if index == _CURRENT:
         index = torch.cuda.current_device()
     h = torch._C._cuda_getCurrentRawStream(index)
     return _LaunchStream(h, index), ctypes.c_void_p(h)
